@@ -751,10 +751,11 @@ extern "C" int nnrh_qconv_create(nnrh_qconv_t* out, const nnrh_qconv_desc* d) {
         if (first_copies) stem_setup(h);
     }
     // scratch: transformed input and row sums (the stem kernel reads the
-    // image itself)
-    if (h->transform == 3 && !h->use_stem && !h->use_stem_f32) {
+    // image itself; stem_scratch allocates the multi-copy image when a run
+    // takes the other path)
+    if (h->transform == 3) {
         size_t bytes = (size_t)(4 >> h->g.copy_shift) * (size_t)h->g.copy_stride;
-        if ((rc = nnrh_malloc((void**)&h->xs, bytes))) return fail(rc);
+        if (!h->use_stem && !h->use_stem_f32 && (rc = nnrh_malloc((void**)&h->xs, bytes))) return fail(rc);
     } else if (h->transform) {
         size_t bytes = (size_t)d->N * d->H * d->W * h->Cx;
         if ((rc = nnrh_malloc((void**)&h->xs, bytes))) return fail(rc);
