@@ -637,13 +637,13 @@ extern "C" int nnrh_qconv_create(nnrh_qconv_t* out, const nnrh_qconv_desc* d) {
             for (int n = 0; n < OCg; ++n) {
                 const int oc = g * OCg + n;
                 const size_t pi = (size_t)g * Np + n;
-                int8_t* row = wp.data() + ((size_t)g * Np + packed_row_of_col(n)) * Kp;
+                int8_t* const wg = wp.data() + (size_t)g * Np * Kp;
                 int32_t s = 0;
                 for (int c = 0; c < Cg; ++c)
                     for (int a = 0; a < d->kH; ++a)
                         for (int b = 0; b < d->kW; ++b) {
                             int8_t v = d->w_host[(((size_t)oc * Cg + c) * d->kH + a) * d->kW + b];
-                            row[(a * kWp + b) * Cgp + c] = v;
+                            wg[packed_off(n, (a * kWp + b) * Cgp + c, Kp)] = v;
                             s += v;
                         }
                 colsum[pi] = s;
@@ -1129,11 +1129,10 @@ extern "C" int nnrh_qmatmul_create(nnrh_qmatmul_t* out, const nnrh_qmatmul_desc*
     std::vector<int32_t> colsum(Np, 0);
     const uint8_t* braw = (const uint8_t*)d->b_host;
     for (int j = 0; j < n; ++j) {
-        int8_t* row = wp.data() + (size_t)packed_row_of_col(j) * Kp;
         int32_t s = 0;
         for (int i = 0; i < k; ++i) {
             int8_t v = (int8_t)(braw[(size_t)i * n + j] ^ (bu8 ? 0x80 : 0));
-            row[i] = v;
+            wp[packed_off(j, i, Kp)] = v;
             s += v;
         }
         colsum[j] = s;
@@ -1237,11 +1236,10 @@ extern "C" int nnrh_matmul_integer_scaled_create(nnrh_qmatmul_t* out, const nnrh
     std::vector<int32_t> colsum(Np, 0);
     const uint8_t* braw = (const uint8_t*)d->b_host;
     for (int j = 0; j < n; ++j) {
-        int8_t* row = wp.data() + (size_t)packed_row_of_col(j) * Kp;
         int32_t sum = 0;
         for (int i = 0; i < k; ++i) {
             const int8_t v = (int8_t)(braw[(size_t)i * n + j] ^ (bu8 ? 0x80 : 0));
-            row[i] = v;
+            wp[packed_off(j, i, Kp)] = v;
             sum += v;
         }
         colsum[j] = sum;
@@ -1421,18 +1419,10 @@ extern "C" int nnrh_qmatmul_fuse_gelu(nnrh_qmatmul_t h) {
     return NNRH_OK;
 }
 
-// (min, max) pairs a fused-dequantize run writes: one per (tile, wave) of the
-// tile the launcher picks for N
-static long long qmatmul_parts(const GemmArgs& g, int batch) {
-    const bool tall = pick_tile(g.N) == TILE_256x64;
-    const int BM = tall ? 256 : 128, BN = tall ? 64 : 128;
-    return (long long)((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN) * batch * 4;
-}
-
 extern "C" int nnrh_qmatmul_minmax_count(nnrh_qmatmul_t h, int batch, int* count) {
     if (!h || !count || batch <= 0) return set_err(NNRH_ERR_INVALID, "qmatmul_minmax_count: bad arguments");
     if (!h->g.dq_bias) return set_err(NNRH_ERR_UNSUPPORTED, "qmatmul_minmax_count: needs nnrh_qmatmul_fuse_dq_bias first");
-    const long long n = qmatmul_parts(h->g, batch);
+    const long long n = qgemm_pairs(h->g, batch);
     if (n > 0x7fffffffLL) return set_err(NNRH_ERR_UNSUPPORTED, "qmatmul_minmax_count: too many tiles");
     *count = (int)n;
     return NNRH_OK;
@@ -1484,7 +1474,7 @@ extern "C" int nnrh_qmatmul_dynamic_quantize_codes(nnrh_qmatmul_t h, const void*
     if (!g.dq_codes || !g.mm_parts || !h->codes_table)
         return set_err(NNRH_ERR_UNSUPPORTED, "qmatmul_dynamic_quantize_codes: needs nnrh_qmatmul_set_minmax_out, "
                                              "then nnrh_qmatmul_set_codes_out");
-    const long long nparts = qmatmul_parts(g, batch);
+    const long long nparts = qgemm_pairs(g, batch);
     if (nparts > h->parts_cap)
         return set_err(NNRH_ERR_INVALID, "qmatmul_dynamic_quantize_codes: %lld min/max pairs exceed the buffer's %d",
                        nparts, h->parts_cap);
@@ -1530,9 +1520,9 @@ extern "C" int nnrh_qmatmul_run(nnrh_qmatmul_t h, const void* a, long long a_bst
     }
     int vec = pick_vec(g.K, (int)g.lda, (uintptr_t)a);
     if (a_bstride % vec) vec = 1;
-    if (g.mm_parts && qmatmul_parts(g, batch) > h->parts_cap)
+    if (g.mm_parts && qgemm_pairs(g, batch) > h->parts_cap)
         return set_err(NNRH_ERR_INVALID, "qmatmul_run: %lld min/max pairs exceed the buffer's %d",
-                       qmatmul_parts(g, batch), h->parts_cap);
+                       qgemm_pairs(g, batch), h->parts_cap);
     ProfScope ps("qgemm", s);
     HIP_TRY(launch_qgemm(g, batch, pick_tile(g.N), vec, s), "qgemm");
     return NNRH_OK;
@@ -1577,9 +1567,9 @@ extern "C" int nnrh_matmul_integer_create(nnrh_matmul_integer_t* out, int m, int
     return NNRH_OK;
 }
 
-int matmul_integer_gemm(nnrh_matmul_integer* h, const void* a, long long a_bstride, const int8_t* bpack,
-                        const int32_t* colsum, bool b_batched, int a_zp, int b_zp, int32_t* y, int batch,
-                        hipStream_t s, const void* a_zp_dev = nullptr);
+static int matmul_integer_any(nnrh_matmul_integer* h, const void* a, long long a_bstride, const void* b,
+                              long long b_bstride, int a_zp, const void* a_zp_dev, int b_zp, int32_t* y, int batch,
+                              hipStream_t s);
 
 extern "C" int nnrh_matmul_integer_run(nnrh_matmul_integer_t h, const void* a, long long a_bstride,
                                        const void* b, long long b_bstride, int a_zp, int b_zp,
@@ -1587,16 +1577,7 @@ extern "C" int nnrh_matmul_integer_run(nnrh_matmul_integer_t h, const void* a, l
     if (!h || !a || !b || !y) return set_err(NNRH_ERR_INVALID, "matmul_integer_run: NULL argument");
     if (batch <= 0 || batch > h->max_batch)
         return set_err(NNRH_ERR_INVALID, "matmul_integer_run: batch %d (max %d)", batch, h->max_batch);
-    hipStream_t s = S(stream);
-    const bool bu8 = h->b_dtype == NNRH_U8;
-    const int nb_b = b_bstride == 0 ? 1 : batch;
-    {
-        ProfScope ps0("pack_b", s);
-        HIP_TRY(launch_pack_b_dense(b, b_bstride, h->k, h->n, h->Kp, h->Np, bu8 ? 0x80 : 0, h->bpack,
-                                    (long long)h->Np * h->Kp, h->colsum, h->Np, nb_b, s),
-                "pack_b");
-    }
-    return matmul_integer_gemm(h, a, a_bstride, h->bpack, h->colsum, b_bstride != 0, a_zp, b_zp, y, batch, s);
+    return matmul_integer_any(h, a, a_bstride, b, b_bstride, a_zp, nullptr, b_zp, y, batch, S(stream));
 }
 
 extern "C" int nnrh_matmul_integer_run_dev_zp(nnrh_matmul_integer_t h, const void* a, long long a_bstride,
@@ -1605,47 +1586,31 @@ extern "C" int nnrh_matmul_integer_run_dev_zp(nnrh_matmul_integer_t h, const voi
     if (!h || !a || !b || !y || !a_zp_dev) return set_err(NNRH_ERR_INVALID, "matmul_integer_run_dev_zp: NULL argument");
     if (batch <= 0 || batch > h->max_batch)
         return set_err(NNRH_ERR_INVALID, "matmul_integer_run_dev_zp: batch %d (max %d)", batch, h->max_batch);
-    hipStream_t s = S(stream);
-    const bool bu8 = h->b_dtype == NNRH_U8;
-    const int nb_b = b_bstride == 0 ? 1 : batch;
-    {
-        ProfScope ps0("pack_b", s);
-        HIP_TRY(launch_pack_b_dense(b, b_bstride, h->k, h->n, h->Kp, h->Np, bu8 ? 0x80 : 0, h->bpack,
-                                    (long long)h->Np * h->Kp, h->colsum, h->Np, nb_b, s),
-                "pack_b");
-    }
-    return matmul_integer_gemm(h, a, a_bstride, h->bpack, h->colsum, b_bstride != 0, 0, b_zp, y, batch, s,
-                               a_zp_dev);
+    return matmul_integer_any(h, a, a_bstride, b, b_bstride, 0, a_zp_dev, b_zp, y, batch, S(stream));
 }
 
-// the GEMM of MatMulInteger over a packed B ([batch][Np][Kp] int8 and its
-// column sums [batch][Np]; one shared when !b_batched)
-int matmul_integer_gemm(nnrh_matmul_integer* h, const void* a, long long a_bstride, const int8_t* bpack,
-                        const int32_t* colsum, bool b_batched, int a_zp, int b_zp, int32_t* y, int batch,
-                        hipStream_t s, const void* a_zp_dev) {
+// B packed per call (one when b_bstride is 0), then the GEMM. The small-tile
+// kernel forms the zero-point sums from the operands it multiplies; the others
+// read them from a pass over B and, with a B zero point, one over A.
+static int matmul_integer_any(nnrh_matmul_integer* h, const void* a, long long a_bstride, const void* b,
+                              long long b_bstride, int a_zp, const void* a_zp_dev, int b_zp, int32_t* y, int batch,
+                              hipStream_t s) {
     const bool au8 = h->a_dtype == NNRH_U8, bu8 = h->b_dtype == NNRH_U8;
+    const bool b_batched = b_bstride != 0;
     GemmArgs g{};
     g.a = (const uint8_t*)a;
     g.lda = h->k;
     g.a_bstride = a_bstride;
     g.a_xor = au8 ? 0x80 : 0;
     g.M = h->m; g.N = h->n; g.K = h->k; g.Kp = h->Kp;
-    g.b = bpack;
+    g.b = h->bpack;
     g.b_bstride = b_batched ? (long long)h->Np * h->Kp : 0;
     g.Np = h->Np;
-    g.colsum = colsum;
     g.param_bstride = b_batched ? h->Np : 0;
     g.a_sub = au8 ? 128 : 0;
     g.alpha = a_zp - g.a_sub;
     g.alpha_zp_dev = a_zp_dev;
     g.beta = b_zp - (bu8 ? 128 : 0);
-    if (g.beta != 0) {
-        HIP_TRY(launch_rowsum_dense((const uint8_t*)a, g.lda, a_bstride, h->m, h->k, !au8, a_zp, a_zp_dev,
-                                    h->rowsum, batch, s),
-                "rowsum_dense");
-        g.rowsum = h->rowsum;
-        g.rowsum_bstride = h->m;
-    }
     g.epi = EPI_I32;
     g.y = y;
     g.ldy = h->n;
@@ -1654,6 +1619,22 @@ int matmul_integer_gemm(nnrh_matmul_integer* h, const void* a, long long a_bstri
     g.bprime_from = h->n;
     int vec = pick_vec(h->k, h->k, (uintptr_t)a);
     if (a_bstride % vec) vec = 1;
+    g.sums_inline = 1;
+    g.colsum = h->colsum;
+    g.rowsum = g.beta != 0 ? h->rowsum : nullptr;
+    g.rowsum_bstride = h->m;
+    g.sums_inline = qgemm_small_eligible(g, batch, vec) ? 1 : 0;
+    {
+        ProfScope ps0("pack_b", s);
+        HIP_TRY(launch_pack_b_dense(b, b_bstride, h->k, h->n, h->Kp, h->Np, bu8 ? 0x80 : 0, h->bpack,
+                                    (long long)h->Np * h->Kp, g.sums_inline ? nullptr : h->colsum, h->Np,
+                                    b_batched ? batch : 1, s),
+                "pack_b");
+    }
+    if (g.rowsum && !g.sums_inline)
+        HIP_TRY(launch_rowsum_dense((const uint8_t*)a, g.lda, a_bstride, h->m, h->k, !au8, a_zp, a_zp_dev,
+                                    h->rowsum, batch, s),
+                "rowsum_dense");
     ProfScope ps("qgemm", s);
     HIP_TRY(launch_qgemm(g, batch, pick_tile(h->n), vec, s), "qgemm");
     return NNRH_OK;
@@ -1808,7 +1789,7 @@ struct nnrh_conv_integer {
     int x_dtype = 0, w_dtype = 0, Kp = 0, Np = 0;
     GemmArgs g{};
     uint8_t* xs = nullptr;        // NHWC copy [N][iH][iW][G * Cgp]
-    int8_t* wpack = nullptr;      // [G][Np][Kp]
+    int8_t* wpack = nullptr;      // [G] x packed_off, Np x Kp bytes each
     int32_t* c0 = nullptr;        // [G][Np]
     int32_t* coef = nullptr;      // [G][Np] row-term coefficient
     ~nnrh_conv_integer() {

@@ -45,13 +45,13 @@ struct GemmArgs {
     long long lda;        // dense row stride (bytes)
     long long a_bstride;  // per-batch stride (blockIdx.z)
     int a_xor;            // 0x80 for uint8 activations (x-128), 0 for int8
-    int M, N, K, Kp;      // K real, Kp = K rounded up to 64 (packed B row length)
+    int M, N, K, Kp;      // K real, Kp = K rounded up to 64 (packed B)
     // conv geometry (A_CONV)
     int H, W, C, oH, oW, kH, kW, sH, sW, dH, dW, pad_t, pad_l;
     int Cs;               // channel stride of the NHWC tensor (>= C; groups)
     int kWp;              // > 0: first-layer layout (kW padded to a multiple of 4)
     int pad_byte;         // raw byte for out-of-image taps (x_zp)
-    // ---- B (weights), packed [Np][Kp] int8 with the 64-column permutation ----
+    // ---- B (weights), packed int8 [Np / 16][Kp / 64] 1 KB pieces (packed_off) ----
     const int8_t* b;
     long long b_bstride;
     int Np;
@@ -73,6 +73,9 @@ struct GemmArgs {
     // the Kp bytes of im2col row m (padding reads pad_byte, which must be the
     // zero point alpha + a_sub) taken from the A fragments in the kernel
     const int32_t* row_coef;
+    // small-tile kernel, EPI_I32: it sums A's rows and B's columns itself (colsum
+    // and rowsum unused)
+    int sums_inline;
     // ---- epilogue ----
     int epi;
     int tail;
@@ -174,6 +177,15 @@ hipError_t launch_qgemm(const GemmArgs& g, int batch, int tile, int vec,
 // pipelined direct-to-LDS variant (nnrh_qgemm_dma.hip) and its eligibility
 bool qgemm_dma_eligible(const GemmArgs& g, int vec);
 hipError_t launch_qgemm_dma(const GemmArgs& g, int batch, int tile, hipStream_t s);
+// (min, max) pairs a fused-dequantize run writes: 4 per tile the pipelined
+// launcher picks for N, one a wave (the small-tile kernel writes as many)
+inline long long qgemm_pairs(const GemmArgs& g, int batch) {
+    const int BM = g.N <= 64 ? 256 : 128, BN = g.N <= 64 ? 64 : 128;
+    return (long long)((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN) * batch * 4;
+}
+// small-tile kernel for grids that leave the chip idle (nnrh_qgemm_small.hip)
+bool qgemm_small_eligible(const GemmArgs& g, int batch, int vec);
+hipError_t launch_qgemm_small(const GemmArgs& g, int batch, int vec, hipStream_t s);
 // barrier-free short-K kernel (nnrh_qgemm_dma.hip): dense A, Kp = 64, RQ-B
 bool qgemm_direct_eligible(const GemmArgs& g, int batch);
 hipError_t launch_qgemm_direct(const GemmArgs& g, hipStream_t s);
@@ -182,7 +194,7 @@ hipError_t launch_qgemm_direct(const GemmArgs& g, hipStream_t s);
 // NCHW fp32 (or uint8) image with C <= 4 channels -> NHWC uint8, RQ-C.
 struct StemArgs {
     const void* x;          // [N][C][H][W] fp32 or uint8
-    const int8_t* w;        // packed weights [64][Kp], K order (kh, kw < 4 * cpr, c < 4)
+    const int8_t* w;        // packed weights (packed_off, 64 columns), K order (kh, kw < 4 * cpr, c < 4)
     const int32_t* c0;      // [64] accumulator start (-(x_zp - 128) * colsum)
     const float* cs;        // [64] RQ-C scale
     const float* bf;        // [64] RQ-C bias term
@@ -279,17 +291,25 @@ struct ConvIntPrepArgs {
     int copy_blocks, vec;   // set by the launcher
 };
 hipError_t launch_conv_integer_prep(ConvIntPrepArgs a, hipStream_t s);
-// Pack a row-major B[K][N] (int8 or uint8) into the kernel's [Np][Kp]
-// permuted layout and compute colsum[n] = sum_k (b - b_sub).
+// Pack a row-major B[K][N] (int8 or uint8) into the kernels' layout
+// (packed_off) and, unless it is NULL, compute colsum[n] = sum_k (b - b_sub).
 hipError_t launch_pack_b_dense(const void* b, long long b_bstride, int K,
                                int N, int Kp, int Np, int b_xor, int8_t* out,
                                long long out_bstride, int32_t* colsum,
                                long long colsum_bstride, int batch,
                                hipStream_t s);
 
-// Row permutation of packed B inside each 64-column group: storage row of
-// logical column n. The MFMA epilogue then sees 16 consecutive columns per
-// lane (see nnrh_qgemm.hip).
+// Packed B: offset of byte (column n < Np, k < Kp). A piece is the operand of
+// one MFMA, 16 consecutive columns x 64 K bytes, one contiguous kilobyte (8
+// whole cache lines; as 16 half lines of a row-major [Np][Kp] the same bytes
+// cost the L1 twice as much); the pieces of a column group follow each other
+// along K.
+__host__ __device__ inline long long packed_off(int n, int k, int Kp) {
+    return (long long)(n >> 4) * Kp * 16 + (long long)(k >> 6) * 1024 + (n & 15) * 64 + (k & 63);
+}
+// Row order of a 64-column tile: MFMA row block tn = row / 16 holds columns
+// 16 g + 4 tn + r at rows 4 g + r, so each lane ends with 16 consecutive
+// columns of one output row (see nnrh_qgemm.hip). Its own inverse.
 __host__ __device__ inline int packed_row_of_col(int n) {
     int g = n >> 6, nl = n & 63;
     int tn = (nl & 15) >> 2;
