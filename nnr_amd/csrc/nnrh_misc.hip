@@ -1042,7 +1042,10 @@ __global__ __launch_bounds__(256) void pack_b_kernel(const uint8_t* __restrict b
 #pragma unroll
                 for (int q = 0; q < 4; ++q) w[q] ^= x;
             } else {
-                for (int i = 0; i < N - n; ++i) w[i >> 2] |= (uint32_t)(p[i] ^ (uint8_t)b_xor) << (8 * (i & 3));
+                // (constant indices: the words stay in registers)
+#pragma unroll
+                for (int i = 0; i < 15; ++i)
+                    if (n + i < N) w[i >> 2] |= (uint32_t)(p[i] ^ (uint8_t)b_xor) << (8 * (i & 3));
             }
         }
         *(uint4*)(tile + (t >> 2) * RS + (t & 3) * 16) = make_uint4(w[0], w[1], w[2], w[3]);
