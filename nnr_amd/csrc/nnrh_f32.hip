@@ -789,16 +789,18 @@ constexpr int MHA_KP = 68;   // K row stride in LDS (floats): rows 16 bytes apar
 // parts (optional): one (min, max) pair per wave, at 2 (4 blockIdx.x + wave),
 // of the values the wave stores (0 stands in for nothing, as for every
 // producer that feeds a DynamicQuantizeLinear, whose range includes 0)
+// TT: key tiles of 16 (8, or 4 / 2 for sequences of at most 64 / 32: a
+// 37-token head took 16.2 us through all 8)
 // CODES: q, k, v given as chain bytes (DqCodes; columns = the hidden axis),
 // each element formed as the producing GEMM's epilogue would have stored it
-template <bool CODES>
+template <bool CODES, int TT>
 __global__ __launch_bounds__(256, 3) void mha_fused_hd64_kernel(const float* __restrict q, const float* __restrict k,
                                                              const float* __restrict v, DqCodes qq, DqCodes kq,
                                                              DqCodes vq, float* __restrict y,
                                                              int S, int Hd, int nh, float scale,
                                                              float* __restrict parts) {
     // one buffer: K (row stride MHA_KP) for the scores, then V (stride 64)
-    __shared__ __attribute__((aligned(16))) float ks[128 * MHA_KP];
+    __shared__ __attribute__((aligned(16))) float ks[16 * TT * MHA_KP];
     float* const vs = ks;
     const int b = blockIdx.x / nh, h = blockIdx.x - b * nh;
     const long long base = (long long)b * S * Hd + (long long)h * 64;
@@ -811,27 +813,27 @@ __global__ __launch_bounds__(256, 3) void mha_fused_hd64_kernel(const float* __r
         else
             return *(const float4*)(x + off);
     };
-    // K: all 8 of a thread's 16-byte pieces in flight before the LDS writes
+    // K: all TT of a thread's 16-byte pieces in flight before the LDS writes
     {
-        float4 kv[8];
+        float4 kv[TT];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < TT; ++j) {
             const int i = threadIdx.x + 256 * j;
             const int t = i >> 4, c = (i & 15) * 4;
             kv[j] = t < S ? load4(k, kq, base + (long long)t * Hd + c, c) : zero4;
         }
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < TT; ++j) {
             const int i = threadIdx.x + 256 * j;
             *(float4*)(ks + (i >> 4) * MHA_KP + (i & 15) * 4) = kv[j];
         }
     }
-    // CODES: V's bytes (4 per dword, 8 dwords a thread) load now, with K's
+    // CODES: V's bytes (4 per dword, TT dwords a thread) load now, with K's
     // and Q's, and become values only when V takes the LDS buffer
-    uint32_t vpre[CODES ? 8 : 1];
+    uint32_t vpre[CODES ? TT : 1];
     if constexpr (CODES) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < TT; ++j) {
             const int i = threadIdx.x + 256 * j;
             const int t = i >> 4, c = (i & 15) * 4;
             vpre[j] = t < S ? *(const uint32_t*)(vq.q + base + (long long)t * Hd + c) : 0u;
@@ -854,9 +856,9 @@ __global__ __launch_bounds__(256, 3) void mha_fused_hd64_kernel(const float* __r
     __syncthreads();
     const bool active = s0 < S;   // a wave with no query still takes every barrier
 
-    f32x4 acc[8][2];
+    f32x4 acc[TT][2];
 #pragma unroll
-    for (int tt = 0; tt < 8; ++tt) {
+    for (int tt = 0; tt < TT; ++tt) {
         acc[tt][0] = f32x4{0.f, 0.f, 0.f, 0.f};
         acc[tt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
         float kf[16];
@@ -877,7 +879,7 @@ __global__ __launch_bounds__(256, 3) void mha_fused_hd64_kernel(const float* __r
     for (int ts = 0; ts < 2; ++ts) {
         float m = -INFINITY;
 #pragma unroll
-        for (int tt = 0; tt < 8; ++tt)
+        for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float x = 16 * tt + 4 * g + i < S ? acc[tt][ts][i] * scale : -INFINITY;
@@ -888,7 +890,7 @@ __global__ __launch_bounds__(256, 3) void mha_fused_hd64_kernel(const float* __r
         m = fmaxf(m, __shfl_xor(m, 32, 64));
         float sum = 0.0f;
 #pragma unroll
-        for (int tt = 0; tt < 8; ++tt)
+        for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float e = expf(acc[tt][ts][i] - m);
@@ -899,7 +901,7 @@ __global__ __launch_bounds__(256, 3) void mha_fused_hd64_kernel(const float* __r
         sum += __shfl_xor(sum, 32, 64);
         const float inv = 1.0f / sum;
 #pragma unroll
-        for (int tt = 0; tt < 8; ++tt)
+        for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
             for (int i = 0; i < 4; ++i) acc[tt][ts][i] = acc[tt][ts][i] * inv;
     }
@@ -907,7 +909,7 @@ __global__ __launch_bounds__(256, 3) void mha_fused_hd64_kernel(const float* __r
     __syncthreads();
     if constexpr (CODES) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < TT; ++j) {
             const int i = threadIdx.x + 256 * j;
             const int t = i >> 4, c = (i & 15) * 4;
             *(float4*)(vs + t * 64 + c) =
@@ -915,7 +917,7 @@ __global__ __launch_bounds__(256, 3) void mha_fused_hd64_kernel(const float* __r
                       : zero4;
         }
     } else {
-        for (int i = threadIdx.x; i < 128 * 16; i += 256) {
+        for (int i = threadIdx.x; i < 16 * TT * 16; i += 256) {
             const int t = i >> 4, c = (i & 15) * 4;
             const long long off = base + (long long)t * Hd + c;
             *(float4*)(vs + t * 64 + c) = t < S ? load4(v, vq, off, c) : zero4;
@@ -933,7 +935,7 @@ __global__ __launch_bounds__(256, 3) void mha_fused_hd64_kernel(const float* __r
 #pragma unroll
         for (int td = 0; td < 4; ++td) o[ts][td] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int tt = 0; tt < 8; ++tt)
+    for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float4 vv = *(const float4*)(vs + (16 * tt + 4 * g + i) * 64 + 4 * lr);
@@ -971,15 +973,217 @@ __global__ __launch_bounds__(256, 3) void mha_fused_hd64_kernel(const float* __r
     }
 }
 
+// ---------------------------------------------------------------------------
+// Attention over any number of keys (head sizes 32, 64, 80, 96, 128): a block
+// takes 64 queries of one (batch, head), 16 a wave, and walks the keys 64 at a
+// time with a running maximum and sum, so the score matrix never leaves
+// registers. fp32 throughout: the matrix unit bounds it (4 S^2 hidden
+// operations a sequence at 154 TFLOP/s; 8 x 512 x 12 heads of 64: 42 us).
+// 64-query blocks rather than 128 balance the chip (8 x 12 heads x 512 queries
+// are 768 blocks, 3 a CU) and let 4 blocks share a CU, so one block's exp()
+// runs under another's MFMAs. The next keys and values load into registers
+// while the current ones multiply.
+// The products use the operand orders of the kernel above: scores as S^T (lane
+// (g, lr) holds keys 16 tt + 4 g + i of query lr), which is the A operand of P
+// V; a lane of O holds queries 4 g + i.
+template <int HD>
+__global__ __launch_bounds__(256, HD <= 64 ? 4 : HD <= 96 ? 3 : 2) void mha_flash_kernel(
+    const float* __restrict q, const float* __restrict k, const float* __restrict v, float* __restrict y, int S,
+    int Hd, int nh, int nqb, int total, float scale) {
+    constexpr int KB = 64;                 // keys a step
+    constexpr int RS = HD + 4;             // LDS row stride (floats): 16 rows apart in the banks
+    constexpr int H4 = HD / 4;             // floats of a row one lane group multiplies
+    constexpr int TD = HD / 16;            // output tiles
+    constexpr bool VEC = HD % 64 == 0;     // lane lr takes columns TD lr + td, else 16 td + lr
+    constexpr int LD = KB * HD / 4 / 256;  // 16-byte pieces of K (or V) a thread moves
+    __shared__ __attribute__((aligned(16))) float ks[KB * RS], vs[KB * RS];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int lr = lane & 15, g = lane >> 4;
+    // the query blocks of a head are neighbours on one XCD (its K and V stay
+    // in that L2)
+    const int per = (total + 7) >> 3;
+    const int t = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || t >= total) return;
+    const int bh = t / nqb, b = bh / nh, h = bh - b * nh;
+    const long long base = (long long)b * S * Hd + (long long)h * HD;
+    const int sq = (t - bh * nqb) * 64 + 16 * w + lr;   // this lane's query (scores)
+    float4 kr[LD], vr[LD];
+    auto fetch = [&](int t0) {
+#pragma unroll
+        for (int j = 0; j < LD; ++j) {
+            const int i = tid + 256 * j, row = i / H4, c = (i - row * H4) * 4;
+            const bool in = t0 + row < S;
+            const long long off = base + (long long)(in ? t0 + row : 0) * Hd + c;
+            kr[j] = *(const float4*)(k + off);
+            vr[j] = *(const float4*)(v + off);
+            if (!in) {   // keys past the end weigh 0 (exp(-inf)): their values must be finite
+                kr[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+                vr[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+        }
+    };
+    auto stage = [&]() {
+#pragma unroll
+        for (int j = 0; j < LD; ++j) {
+            const int i = tid + 256 * j, row = i / H4, c = (i - row * H4) * 4;
+            *(float4*)(ks + row * RS + c) = kr[j];
+            *(float4*)(vs + row * RS + c) = vr[j];
+        }
+    };
+    fetch(0);
+    float qf[H4];
+    {
+        const float* qr = q + base + (long long)(sq < S ? sq : S - 1) * Hd + g * H4;
+#pragma unroll
+        for (int j = 0; j < H4; j += 4) {
+            const float4 x = *(const float4*)(qr + j);
+            qf[j] = x.x; qf[j + 1] = x.y; qf[j + 2] = x.z; qf[j + 3] = x.w;
+        }
+    }
+    f32x4 o[TD];
+#pragma unroll
+    for (int td = 0; td < TD; ++td) o[td] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.0f;   // of query lr (the same in the 4 lane groups)
+    stage();
+    for (int t0 = 0; t0 < S; t0 += KB) {
+        __syncthreads();
+        const bool more = t0 + KB < S;
+        if (more) fetch(t0 + KB);
+        f32x4 p[4];
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) {
+            p[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            const float* kp = ks + (16 * tt + lr) * RS + g * H4;
+#pragma unroll
+            for (int j = 0; j < H4; j += 4) {
+                const float4 x = *(const float4*)(kp + j);
+                p[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, qf[j], p[tt], 0, 0, 0);
+                p[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, qf[j + 1], p[tt], 0, 0, 0);
+                p[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.z, qf[j + 2], p[tt], 0, 0, 0);
+                p[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w, qf[j + 3], p[tt], 0, 0, 0);
+            }
+        }
+        float bm = -INFINITY;
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float x = t0 + 16 * tt + 4 * g + i < S ? p[tt][i] * scale : -INFINITY;
+                p[tt][i] = x;
+                bm = fmaxf(bm, x);
+            }
+        bm = fmaxf(bm, __shfl_xor(bm, 16, 64));
+        bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
+        const float mn = fmaxf(m, bm);
+        // (every score so far -inf: exp(-inf - 0) = 0, not exp(-inf + inf))
+        const float mu = mn == -INFINITY ? 0.0f : mn;
+        const float alpha = expf(m - mu);
+        m = mn;
+        float sum = 0.0f;
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float e = expf(p[tt][i] - mu);
+                p[tt][i] = e;
+                sum += e;
+            }
+        sum += __shfl_xor(sum, 16, 64);
+        sum += __shfl_xor(sum, 32, 64);
+        l = l * alpha + sum;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float a = __shfl(alpha, 4 * g + i, 64);
+#pragma unroll
+            for (int td = 0; td < TD; ++td) o[td][i] *= a;
+        }
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float* vp = vs + (16 * tt + 4 * g + i) * RS;
+                float vb[TD];
+                if constexpr (VEC) {
+#pragma unroll
+                    for (int j = 0; j < TD; j += 4) {
+                        const float4 x = *(const float4*)(vp + TD * lr + j);
+                        vb[j] = x.x; vb[j + 1] = x.y; vb[j + 2] = x.z; vb[j + 3] = x.w;
+                    }
+                } else {
+#pragma unroll
+                    for (int td = 0; td < TD; ++td) vb[td] = vp[16 * td + lr];
+                }
+#pragma unroll
+                for (int td = 0; td < TD; ++td)
+                    o[td] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[tt][i], vb[td], o[td], 0, 0, 0);
+            }
+        if (more) {
+            __syncthreads();   // every wave is done with the keys in LDS
+            stage();
+        }
+    }
+    const float inv = 1.0f / l;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float a = __shfl(inv, 4 * g + i, 64);
+        const int s = (t - bh * nqb) * 64 + 16 * w + 4 * g + i;
+        if (s >= S) continue;
+        float* yp = y + base + (long long)s * Hd;
+        if constexpr (VEC) {
+#pragma unroll
+            for (int j = 0; j < TD; j += 4)
+                *(float4*)(yp + TD * lr + j) =
+                    make_float4(o[j][i] * a, o[j + 1][i] * a, o[j + 2][i] * a, o[j + 3][i] * a);
+        } else {
+#pragma unroll
+            for (int td = 0; td < TD; ++td) yp[16 * td + lr] = o[td][i] * a;
+        }
+    }
+}
+
+// false: a shape or alignment the kernel does not take
+static bool launch_mha_flash(const float* q, const float* k, const float* v, float* y, int B, int S, int Hd, int nh,
+                             float scale, hipStream_t s) {
+    const uintptr_t al = (uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)y;
+    const int nqb = (S + 63) / 64;
+    const long long total = (long long)B * nh * nqb;
+    if ((al & 15) || total > 0x7ffffff0LL) return false;
+    // an output over the keys, or over other rows of the queries: one block
+    // would write what another still reads
+    const size_t n = (size_t)B * S * Hd;
+    auto over = [&](const float* x) { return y < x + n && x < y + n; };
+    if (over(k) || (over(q) && y != q)) return false;
+    const dim3 grid((unsigned)(8 * ((total + 7) / 8)));
+    switch (Hd / nh) {
+#define NNRH_FLASH_CASE(HD)                                                                                        \
+    case HD:                                                                                                       \
+        hipLaunchKernelGGL(mha_flash_kernel<HD>, grid, dim3(256), 0, s, q, k, v, y, S, Hd, nh, nqb, (int)total, \
+                           scale);                                                                                 \
+        return true;
+        NNRH_FLASH_CASE(32) NNRH_FLASH_CASE(64) NNRH_FLASH_CASE(80) NNRH_FLASH_CASE(96) NNRH_FLASH_CASE(128)
+#undef NNRH_FLASH_CASE
+    default: return false;
+    }
+}
+
+template <bool CODES>
+static hipError_t launch_mha_hd64(const float* q, const float* k, const float* v, const DqCodes& qq, const DqCodes& kq,
+                                  const DqCodes& vq, float* y, int B, int S, int Hd, int nh, float scale,
+                                  float* parts, hipStream_t s) {
+    auto kern = S > 64 ? mha_fused_hd64_kernel<CODES, 8>
+                       : (S > 32 ? mha_fused_hd64_kernel<CODES, 4> : mha_fused_hd64_kernel<CODES, 2>);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(B * nh)), dim3(256), 0, s, q, k, v, qq, kq, vq, y, S, Hd, nh, scale,
+                       parts);
+    return hipGetLastError();
+}
+
 hipError_t launch_mha_codes_f32(const DqCodes& q, const DqCodes& k, const DqCodes& v, float* y, int B, int S,
                                 int Hd, int nh, float scale, float* parts, hipStream_t s) {
     if (B <= 0 || S <= 0) return hipSuccess;
     const uintptr_t a4 = (uintptr_t)q.q | (uintptr_t)k.q | (uintptr_t)v.q;
     const uintptr_t a16 = (uintptr_t)y | (uintptr_t)q.bias | (uintptr_t)k.bias | (uintptr_t)v.bias;
     if (!mha_fused_shape(S, Hd, nh) || (a4 & 3) || (a16 & 15)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(mha_fused_hd64_kernel<true>, dim3((unsigned)(B * nh)), dim3(256), 0, s, nullptr, nullptr,
-                       nullptr, q, k, v, y, S, Hd, nh, scale, parts);
-    return hipGetLastError();
+    return launch_mha_hd64<true>(nullptr, nullptr, nullptr, q, k, v, y, B, S, Hd, nh, scale, parts, s);
 }
 
 int mha_minmax_pairs(int B, int S, int Hd, int nh) {
@@ -1001,13 +1205,13 @@ hipError_t launch_mha_f32(const float* q, const float* k, const float* v, float*
     if (nh <= 0 || Hd % nh) return hipErrorInvalidValue;
     if (mha_fused_ok(q, k, v, y, S, Hd, nh)) {
         const DqCodes none{nullptr, 0, 0.0f, nullptr};
-        hipLaunchKernelGGL(mha_fused_hd64_kernel<false>, dim3((unsigned)(B * nh)), dim3(256), 0, s, q, k, v, none,
-                           none, none, y, S, Hd, nh, scale, parts);
-        return hipGetLastError();
+        return launch_mha_hd64<false>(q, k, v, none, none, none, y, B, S, Hd, nh, scale, parts, s);
     }
     if (parts) return hipErrorInvalidValue;   // only the fused kernel writes min / max pairs
-    // scores = Q_h K_h^T per (batch, head), the scaled softmax, then P V_h,
-    // with the heads read and written in place through strides
+    if (launch_mha_flash(q, k, v, y, B, S, Hd, nh, scale, s)) return hipGetLastError();
+    // other head sizes and alignments: scores = Q_h K_h^T per (batch, head),
+    // the scaled softmax, then P V_h, with the heads read and written in place
+    // through strides
     const int hd = Hd / nh;
     float* scores = (float*)ws;
     GemmF32Gen p{};
