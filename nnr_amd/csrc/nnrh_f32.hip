@@ -104,10 +104,44 @@ __global__ __launch_bounds__(256) void gap_dq_nhwc4_kernel(const uint8_t* __rest
         make_float4(s[0] / (float)HW, s[1] / (float)HW, s[2] / (float)HW, s[3] / (float)HW);
 }
 
+// one channel per thread, 64 threads a block and 32 pixels' loads in flight,
+// for grids of a few images: the latency of a thread's loads and its chain of
+// sums bound it (1 x 49 x 2048: two blocks of four channels a thread took 8.2
+// us). The same sum in the same pixel order
+__global__ __launch_bounds__(64) void gap_dq_nhwc1_kernel(const uint8_t* __restrict x, float* __restrict y, int N,
+                                                          int C, int HW, int sgn, float zpf, float sc) {
+    const long long row = (long long)blockIdx.x * 64 + threadIdx.x;
+    if (row >= (long long)N * C) return;
+    const int n = (int)(row / C);
+    const uint8_t* p = x + (long long)n * HW * C + (row - (long long)n * C);
+    float s = 0.0f;
+    for (int i = 0; i < HW; i += 32) {
+        uint32_t q[32];
+#pragma unroll
+        for (int u = 0; u < 32; ++u) q[u] = p[(long long)min(i + u, HW - 1) * C];
+#pragma unroll
+        for (int u = 0; u < 32; ++u) {
+            const float f = sgn ? (float)(int)(int8_t)q[u] : (float)q[u];
+            const float t = s + (f - zpf) * sc;
+            s = i + u < HW ? t : s;
+        }
+    }
+    y[row] = s / (float)HW;
+}
+
+// outputs up to which a thread takes one channel: 1024 waves of them, where
+// four channels a thread make 64 blocks
+constexpr long long GAP_ONE_MAX = 65536;
+
 hipError_t launch_gap_dq(const uint8_t* x, float* y, int N, int C, int HW, int x_nhwc, int x_signed,
                          float scale, int zp, hipStream_t s) {
     const long long rows = (long long)N * C;
     if (rows <= 0) return hipSuccess;
+    if (x_nhwc && HW > 0 && rows <= GAP_ONE_MAX) {
+        hipLaunchKernelGGL(gap_dq_nhwc1_kernel, dim3((unsigned)((rows + 63) / 64)), dim3(64), 0, s, x, y, N, C, HW,
+                           x_signed, (float)zp, scale);
+        return hipGetLastError();
+    }
     if (x_nhwc && (C & 3) == 0 && (((uintptr_t)x | (uintptr_t)y) & 15) == 0) {
         const long long th = rows / 4;
         hipLaunchKernelGGL(gap_dq_nhwc4_kernel, dim3((unsigned)((th + 255) / 256)), dim3(256), 0, s, x, y, N, C,
@@ -139,38 +173,47 @@ hipError_t launch_gap_f32(const float* x, float* y, int N, int C, int HW, int x_
 
 // Small fp32 GEMMs (too few 64x64 tiles to fill the chip, e.g. a
 // classifier over one batch): Y = alpha * A[M][K] . op(B) + beta * Cb with
-// fp32 MFMA 16x16x4. A block computes 32x32 outputs; its 4 waves take every
-// 4th 64-wide K chunk and their partial sums are added in LDS in wave order.
-// Within a chunk the contraction runs over k = 16 (l / 16) + step, so each
-// lane reads 16 consecutive floats of its A row (and of its B row when B is
-// stored [N][K]); rows and columns past M / N read a clamped row and are not
-// stored.
+// fp32 MFMA 16x16x4. A block computes 16 T x 16 T outputs; its W waves take
+// every W-th 64-wide K chunk and their partial sums are added in LDS in wave
+// order. Within a chunk the contraction runs over k = 16 (l / 16) + step, so
+// each lane reads 16 consecutive floats of its A row (and of its B row when B
+// is stored [N][K]); rows and columns past M / N read a clamped row and are
+// not stored. T = 2 with 4 waves reads each operand once per 32 outputs; with
+// few of those tiles the chain of one wave's chunks bounds it (1 x 1000 x
+// 2048: 32 blocks of 8 chunks a wave), so T = 1 with 16 waves takes them
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-template <int TB>
-__global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restrict A, const float* __restrict B,
-                                                            const float* __restrict C, float* __restrict Y, int M,
-                                                            int N, int K, float alpha, float beta, int c_mode) {
-    __shared__ float red[3][32 * 32];
+template <int TB, int T, int W>
+__global__ __launch_bounds__(64 * W) void gemm_f32_mfma_kernel(const float* __restrict A, const float* __restrict B,
+                                                               const float* __restrict C, float* __restrict Y, int M,
+                                                               int N, int K, float alpha, float beta, int c_mode) {
+    __shared__ f32x4 red[W - 1][T * T][64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int lr = lane & 15, g = lane >> 4;
-    const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
-    const float* ar[2] = {A + (long long)min(m0 + lr, M - 1) * K, A + (long long)min(m0 + 16 + lr, M - 1) * K};
-    const int bn[2] = {min(n0 + lr, N - 1), min(n0 + 16 + lr, N - 1)};
-    f32x4 acc[2][2];
+    const int m0 = blockIdx.y * 16 * T, n0 = blockIdx.x * 16 * T;
+    const float* ar[T];
+    int bn[T];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) acc[i][0] = acc[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-    auto load = [&](int c, float (&a)[2][16], float (&b)[2][16]) {
+    for (int t = 0; t < T; ++t) {
+        ar[t] = A + (long long)min(m0 + 16 * t + lr, M - 1) * K;
+        bn[t] = min(n0 + 16 * t + lr, N - 1);
+    }
+    f32x4 acc[T][T];
+#pragma unroll
+    for (int i = 0; i < T; ++i)
+#pragma unroll
+        for (int j = 0; j < T; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto load = [&](int c, float (&a)[T][16], float (&b)[T][16]) {
         const int k0 = c * 64 + 16 * g;
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < T; ++t)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const float4 v = *(const float4*)(ar[t] + k0 + 4 * j);
                 a[t][4 * j] = v.x; a[t][4 * j + 1] = v.y; a[t][4 * j + 2] = v.z; a[t][4 * j + 3] = v.w;
             }
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
+        for (int t = 0; t < T; ++t) {
             if (TB) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
@@ -183,50 +226,47 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
             }
         }
     };
-    auto mma = [&](const float (&a)[2][16], const float (&b)[2][16]) {
+    auto mma = [&](const float (&a)[T][16], const float (&b)[T][16]) {
 #pragma unroll
         for (int st = 0; st < 16; ++st)
 #pragma unroll
-            for (int mt = 0; mt < 2; ++mt)
+            for (int mt = 0; mt < T; ++mt)
 #pragma unroll
-                for (int nt = 0; nt < 2; ++nt)
+                for (int nt = 0; nt < T; ++nt)
                     acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[mt][st], b[nt][st], acc[mt][nt], 0, 0, 0);
     };
     const int nch = K >> 6;
-    float a0[2][16], b0[2][16], a1[2][16], b1[2][16];
+    float a0[T][16], b0[T][16], a1[T][16], b1[T][16];
     int c = w;
     if (c < nch) load(c, a0, b0);
-    for (; c < nch; c += 8) {
+    for (; c < nch; c += 2 * W) {
         // the next chunk's loads are in flight while this one multiplies
-        if (c + 4 < nch) load(c + 4, a1, b1);
+        if (c + W < nch) load(c + W, a1, b1);
         mma(a0, b0);
-        if (c + 4 >= nch) break;
-        if (c + 8 < nch) load(c + 8, a0, b0);
+        if (c + W >= nch) break;
+        if (c + 2 * W < nch) load(c + 2 * W, a0, b0);
         mma(a1, b1);
     }
     // acc[mt][nt][i] = partial Y[m0 + 16 mt + 4 g + i][n0 + 16 nt + lr]
     if (w > 0) {
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
+        for (int mt = 0; mt < T; ++mt)
 #pragma unroll
-            for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) red[w - 1][(16 * mt + 4 * g + i) * 32 + 16 * nt + lr] = acc[mt][nt][i];
+            for (int nt = 0; nt < T; ++nt) red[w - 1][mt * T + nt][lane] = acc[mt][nt];
     }
     __syncthreads();
     if (w > 0) return;
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
+    for (int mt = 0; mt < T; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt)
+        for (int nt = 0; nt < T; ++nt) {
+            f32x4 sum = acc[mt][nt];
+#pragma unroll
+            for (int p = 0; p < W - 1; ++p) sum += red[p][mt * T + nt][lane];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int r = 16 * mt + 4 * g + i, cl = 16 * nt + lr;
-                const int m = m0 + r, n = n0 + cl;
-                float v = acc[mt][nt][i];
-                v = v + red[0][r * 32 + cl];
-                v = v + red[1][r * 32 + cl];
-                v = v + red[2][r * 32 + cl];
+                const int m = m0 + 16 * mt + 4 * g + i, n = n0 + 16 * nt + lr;
+                float v = sum[i];
                 if (m >= M || n >= N) continue;
                 v = alpha * v;
                 if (c_mode != 0 && beta != 0.0f) {
@@ -238,6 +278,7 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
                 }
                 Y[(long long)m * N + n] = v;
             }
+        }
 }
 
 // Any fp32 GEMM: Y(z)[m][n] = alpha * sum_k A(z)(m, k) B(z)(k, n) (+ beta *
@@ -335,13 +376,14 @@ hipError_t launch_gemm_f32_batched(const float* A, const float* B, const float* 
     const long long tiles64 = (long long)((M + 63) / 64) * ((N + 63) / 64);
     if (batch == 1 && !transA && K > 0 && (K & 63) == 0 && tiles64 < 512 && M <= 65535 * 32 &&
         (((uintptr_t)A | (uintptr_t)B) & 15) == 0) {
-        const dim3 grid((unsigned)((N + 31) / 32), (unsigned)((M + 31) / 32));
-        if (transB)
-            hipLaunchKernelGGL(gemm_f32_mfma_kernel<1>, grid, dim3(256), 0, s, A, B, C, Y, M, N, K, alpha, beta,
-                               c_mode);
-        else
-            hipLaunchKernelGGL(gemm_f32_mfma_kernel<0>, grid, dim3(256), 0, s, A, B, C, Y, M, N, K, alpha, beta,
-                               c_mode);
+        // 32 x 32 tiles from 65 of them: 64 leave 252 blocks of 16 x 16 (a
+        // block a CU), more are that many fewer reads of each operand
+        const long long t32 = (long long)((M + 31) / 32) * ((N + 31) / 32);
+        const int bt = t32 <= 64 ? 16 : 32;
+        const dim3 grid((unsigned)((N + bt - 1) / bt), (unsigned)((M + bt - 1) / bt));
+        auto kern = bt == 16 ? (transB ? gemm_f32_mfma_kernel<1, 1, 16> : gemm_f32_mfma_kernel<0, 1, 16>)
+                             : (transB ? gemm_f32_mfma_kernel<1, 2, 4> : gemm_f32_mfma_kernel<0, 2, 4>);
+        hipLaunchKernelGGL(kern, grid, dim3(bt == 16 ? 1024 : 256), 0, s, A, B, C, Y, M, N, K, alpha, beta, c_mode);
         return hipGetLastError();
     }
     // every other shape: the general kernel (A [M][K] or, transposed,

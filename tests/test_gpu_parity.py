@@ -578,6 +578,16 @@ def test_gemm_f32(dev, ta, tb, c_mode, M, N, K):
     np.testing.assert_allclose(to_np(y), ref, atol=1e-3, rtol=1e-4)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1000, 2048),    # 16 x 16 tiles: two K chunks a wave
+                                   (9, 1000, 1280), (16, 17, 1088),   # 17 chunks over 16 waves
+                                   (1, 1, 64), (17, 15, 2112),   # one chunk; 33
+                                   (64, 1000, 128),   # the last grid of 16 x 16 tiles
+                                   (65, 1000, 128)])  # the first of 32 x 32
+@pytest.mark.parametrize("tb,c_mode", [(0, 3), (1, 2)])
+def test_gemm_f32_small_grids(dev, tb, c_mode, M, N, K):
+    test_gemm_f32(dev, 0, tb, c_mode, M, N, K)
+
+
 @pytest.mark.parametrize("ta,tb,shared", [(0, 0, False), (1, 0, True), (0, 1, False), (1, 1, True)])
 def test_gemm_f32_batched(dev, ta, tb, shared):
     """Batched MatMul on the general strided kernel: per-batch A, B per batch
@@ -1132,6 +1142,27 @@ def test_global_avgpool_dequant(dev, nhwc, dt, C):
     deq = O.dequantize_linear(q, s, z)
     ref = deq.mean(axis=(1, 2) if nhwc else (2, 3), dtype=np.float64)
     np.testing.assert_allclose(got, ref, rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("N,C,HW", [(1, 3, 1), (2, 65, 31), (1, 2048, 32), (3, 70, 33), (1, 64, 65),   # one channel a thread
+                                    (32, 2048, 49), (33, 2048, 49), (33, 2050, 33)])   # its last size; past it
+@pytest.mark.parametrize("dt", [np.uint8, np.int8])
+def test_global_avgpool_dequant_sizes(dev, N, C, HW, dt):
+    """NHWC at the edges of the 32-pixel steps and of the output count up to
+    which a thread takes one channel: fp32 sums in pixel order, so a float32
+    running sum gives the same bits."""
+    import torch
+    from nnr_amd import _lib
+    q = np.random.default_rng(N + C + HW).integers(np.iinfo(dt).min, np.iinfo(dt).max + 1, (N, HW, C), dtype=dt)
+    s, z = np.float32(0.0371), np.float32(9 if dt == np.uint8 else -4)
+    qd, y = to_dev(q, dev), torch.empty((N, C), dtype=torch.float32, device=dev)
+    _lib.check(_lib.lib().nnrh_global_avgpool_dequant(_lib.ptr(qd), _lib.ptr(y), N, C, HW, 1,
+                                                      H.U8 if dt == np.uint8 else H.S8, float(s), int(z),
+                                                      _lib.cur_stream()))
+    acc = np.zeros((N, C), np.float32)
+    for i in range(HW):
+        acc = acc + (q[:, i].astype(np.float32) - z) * s
+    assert np.array_equal(to_np(y).view(np.uint32), (acc / np.float32(HW)).view(np.uint32))
 
 
 # ---------------------------------------------------------------------------
