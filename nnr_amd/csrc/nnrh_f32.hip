@@ -832,7 +832,9 @@ constexpr int MHA_KP = 68;   // K row stride in LDS (floats): rows 16 bytes apar
 // of the values the wave stores (0 stands in for nothing, as for every
 // producer that feeds a DynamicQuantizeLinear, whose range includes 0)
 // TT: key tiles of 16 (8, or 4 / 2 for sequences of at most 64 / 32: a
-// 37-token head took 16.2 us through all 8)
+// 37-token head took 16.2 us through all 8). Up to 64 queries a wave takes 16
+// of them and not 32, so that twice the waves share the head (37 tokens, 12
+// heads: 11.3 -> 8.1 us)
 // CODES: q, k, v given as chain bytes (DqCodes; columns = the hidden axis),
 // each element formed as the producing GEMM's epilogue would have stored it
 template <bool CODES, int TT>
@@ -841,6 +843,7 @@ __global__ __launch_bounds__(256, 3) void mha_fused_hd64_kernel(const float* __r
                                                              DqCodes vq, float* __restrict y,
                                                              int S, int Hd, int nh, float scale,
                                                              float* __restrict parts) {
+    constexpr int TS = TT == 8 ? 2 : 1;   // query tiles of a wave
     // one buffer: K (row stride MHA_KP) for the scores, then V (stride 64)
     __shared__ __attribute__((aligned(16))) float ks[16 * TT * MHA_KP];
     float* const vs = ks;
@@ -883,11 +886,11 @@ __global__ __launch_bounds__(256, 3) void mha_fused_hd64_kernel(const float* __r
     }
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int lr = lane & 15, g = lane >> 4;
-    const int s0 = 32 * w;   // this wave's first query
-    // Q[s][16 g .. 16 g + 15] of the wave's two query tiles
-    float qf[2][16];
+    const int s0 = 16 * TS * w;   // this wave's first query
+    // Q[s][16 g .. 16 g + 15] of the wave's query tiles
+    float qf[TS][16];
 #pragma unroll
-    for (int ts = 0; ts < 2; ++ts) {
+    for (int ts = 0; ts < TS; ++ts) {
         const int sq = s0 + 16 * ts + lr;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -898,11 +901,11 @@ __global__ __launch_bounds__(256, 3) void mha_fused_hd64_kernel(const float* __r
     __syncthreads();
     const bool active = s0 < S;   // a wave with no query still takes every barrier
 
-    f32x4 acc[TT][2];
+    f32x4 acc[TT][TS];
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) {
-        acc[tt][0] = f32x4{0.f, 0.f, 0.f, 0.f};
-        acc[tt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ts = 0; ts < TS; ++ts) acc[tt][ts] = f32x4{0.f, 0.f, 0.f, 0.f};
         float kf[16];
         const float* kr = ks + (16 * tt + lr) * MHA_KP + 16 * g;
 #pragma unroll
@@ -911,14 +914,14 @@ __global__ __launch_bounds__(256, 3) void mha_fused_hd64_kernel(const float* __r
             kf[4 * j] = t4.x; kf[4 * j + 1] = t4.y; kf[4 * j + 2] = t4.z; kf[4 * j + 3] = t4.w;
         }
 #pragma unroll
-        for (int st = 0; st < 16; ++st) {
-            acc[tt][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[st], qf[0][st], acc[tt][0], 0, 0, 0);
-            acc[tt][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[st], qf[1][st], acc[tt][1], 0, 0, 0);
-        }
+        for (int st = 0; st < 16; ++st)
+#pragma unroll
+            for (int ts = 0; ts < TS; ++ts)
+                acc[tt][ts] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[st], qf[ts][st], acc[tt][ts], 0, 0, 0);
     }
     // softmax over t of fl(score * scale), per query column
 #pragma unroll
-    for (int ts = 0; ts < 2; ++ts) {
+    for (int ts = 0; ts < TS; ++ts) {
         float m = -INFINITY;
 #pragma unroll
         for (int tt = 0; tt < TT; ++tt)
@@ -971,9 +974,9 @@ __global__ __launch_bounds__(256, 3) void mha_fused_hd64_kernel(const float* __r
         return;
     }
     // O[s][d] = sum_t P[s][t] V[t][d]; output tile td holds d = 4 (l % 16) + td
-    f32x4 o[2][4];
+    f32x4 o[TS][4];
 #pragma unroll
-    for (int ts = 0; ts < 2; ++ts)
+    for (int ts = 0; ts < TS; ++ts)
 #pragma unroll
         for (int td = 0; td < 4; ++td) o[ts][td] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -983,7 +986,7 @@ __global__ __launch_bounds__(256, 3) void mha_fused_hd64_kernel(const float* __r
             const float4 vv = *(const float4*)(vs + (16 * tt + 4 * g + i) * 64 + 4 * lr);
             const float vb[4] = {vv.x, vv.y, vv.z, vv.w};
 #pragma unroll
-            for (int ts = 0; ts < 2; ++ts)
+            for (int ts = 0; ts < TS; ++ts)
 #pragma unroll
                 for (int td = 0; td < 4; ++td)
                     o[ts][td] = __builtin_amdgcn_mfma_f32_16x16x4f32(acc[tt][ts][i], vb[td], o[ts][td], 0, 0, 0);
@@ -991,7 +994,7 @@ __global__ __launch_bounds__(256, 3) void mha_fused_hd64_kernel(const float* __r
     // o[ts][td][i] = O[s0 + 16 ts + 4 g + i][4 lr + td]
     float mn = 0.0f, mx = 0.0f;
 #pragma unroll
-    for (int ts = 0; ts < 2; ++ts)
+    for (int ts = 0; ts < TS; ++ts)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int sq = s0 + 16 * ts + 4 * g + i;

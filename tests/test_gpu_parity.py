@@ -797,7 +797,7 @@ def test_layernorm_codes(dev, rows, D, side):
     assert np.array_equal(to_np(p1).view(np.uint32), to_np(p0).view(np.uint32))
 
 
-@pytest.mark.parametrize("B,S", [(3, 128), (2, 77)])
+@pytest.mark.parametrize("B,S", [(3, 128), (2, 77), (2, 65), (1, 64), (3, 33), (2, 32), (1, 17), (1, 1)])
 def test_mha_codes(dev, B, S):
     """The fused attention reading q, k and v as the uint8 bytes of three
     fused dequantize chains: y and its (min, max) pairs equal, bit for bit,
@@ -1207,6 +1207,10 @@ def test_qconv1d(dev, case):
     (3, 50, 128, 2, 0.3),         # fused, padded key rows and idle waves
     (2, 1, 64, 1, 0.5),           # fused, one token
     (1, 97, 192, 3, -0.7),        # fused, negative scale
+    (2, 64, 128, 2, 0.3),         # fused, 16 queries a wave: all of them; a
+    (1, 65, 128, 2, 0.3),         # key past it; edges of its 16-query waves
+    (2, 33, 128, 2, 0.3),         # and of its key tiles
+    (1, 17, 64, 1, 0.3),
 ])
 def test_multihead_attention_f32(dev, B, S, hidden, heads, scale):
     """MultiHeadAttention (heads read and written in place; the fused fp32
