@@ -1008,6 +1008,11 @@ QFIRST_CASES = [
     # overflow the staging area although a 3-row span (23,040 B) fits: the
     # multi-copy GEMM path runs it
     ("stem_s5_w640", 1, 3, 12, 640, 16, 3, 5, (1, 1, 1, 1), 0.0213, 128),
+    # the number of images from which a strip has several row groups (2 groups
+    # each here), and one fewer: one group, of fewer rows
+    ("rn50_n256", 256, 3, 40, 36, 64, 7, 2, (3, 3, 3, 3), 0.0187, 114),
+    ("rn50_n255", 255, 3, 40, 36, 64, 7, 2, (3, 3, 3, 3), 0.0187, 114),
+    ("mbv2_n9", 9, 3, 112, 112, 32, 3, 2, (1, 1, 1, 1), 0.0237, 131),
 ]
 
 # the first-layer cases the one-kernel stem must take (True) or refuse
@@ -1059,6 +1064,9 @@ QPOOL_CASES = [
     # odd conv output height (the last pooled row's third conv row is
     # padding), 48 channels
     ("odd_rows_f32", 1, 3, 42, 36, 48, True, 9),
+    # strips of several groups (128 images), and one image fewer: of one
+    ("n128_f32", 128, 3, 40, 36, 64, True, 0),
+    ("n127_f32", 127, 3, 40, 36, 64, True, 0),
 ]
 
 
