@@ -106,8 +106,8 @@ __global__ __launch_bounds__(256) void gap_dq_nhwc4_kernel(const uint8_t* __rest
 
 // one channel per thread, 64 threads a block and 32 pixels' loads in flight,
 // for grids of a few images: the latency of a thread's loads and its chain of
-// sums bound it (1 x 49 x 2048: two blocks of four channels a thread took 8.2
-// us). The same sum in the same pixel order
+// sums bound it (1 x 49 x 2048: two blocks of four channels a thread took 8.8
+// us, 32 of one 4.5). The same sum in the same pixel order
 __global__ __launch_bounds__(64) void gap_dq_nhwc1_kernel(const uint8_t* __restrict x, float* __restrict y, int N,
                                                           int C, int HW, int sgn, float zpf, float sc) {
     const long long row = (long long)blockIdx.x * 64 + threadIdx.x;
@@ -180,7 +180,8 @@ hipError_t launch_gap_f32(const float* x, float* y, int N, int C, int HW, int x_
 // is stored [N][K]); rows and columns past M / N read a clamped row and are
 // not stored. T = 2 with 4 waves reads each operand once per 32 outputs; with
 // few of those tiles the chain of one wave's chunks bounds it (1 x 1000 x
-// 2048: 32 blocks of 8 chunks a wave), so T = 1 with 16 waves takes them
+// 2048: 32 blocks of 8 chunks a wave 14.7 us), so T = 1 with 16 waves takes them
+// (63 blocks of 2 chunks a wave, 7.5; 9 x 1000 x 1280 12.4 -> 7.2)
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 template <int TB, int T, int W>
