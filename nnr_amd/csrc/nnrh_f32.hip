@@ -189,15 +189,22 @@ __global__ __launch_bounds__(64 * W) void gemm_f32_mfma_kernel(const float* __re
                                                                const float* __restrict C, float* __restrict Y, int M,
                                                                int N, int K, float alpha, float beta, int c_mode) {
     __shared__ f32x4 red[W - 1][T * T][64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int w = TB || T == 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : (int)(threadIdx.x >> 6);
     const int lr = lane & 15, g = lane >> 4;
     const int m0 = blockIdx.y * 16 * T, n0 = blockIdx.x * 16 * T;
     const float* ar[T];
     int bn[T];
+    // B stored [K][N], T = 1: a wave-uniform row and the lane's offset (16 row
+    // addresses a lane spill 326 registers at the 128 of 16 waves: 1 x 1000 x
+    // 1280 39.7 us, 5.3 so). T = 2 keeps its row addresses in 256 registers
+    // (256 x 2048 x 1280 25.2 us, with the offset 28.3)
+    uint32_t bo[T];
 #pragma unroll
     for (int t = 0; t < T; ++t) {
         ar[t] = A + (long long)min(m0 + 16 * t + lr, M - 1) * K;
         bn[t] = min(n0 + 16 * t + lr, N - 1);
+        bo[t] = (uint32_t)(16 * g) * (uint32_t)N + (uint32_t)bn[t];
     }
     f32x4 acc[T][T];
 #pragma unroll
@@ -223,7 +230,8 @@ __global__ __launch_bounds__(64 * W) void gemm_f32_mfma_kernel(const float* __re
                 }
             } else {
 #pragma unroll
-                for (int st = 0; st < 16; ++st) b[t][st] = B[(long long)(k0 + st) * N + bn[t]];
+                for (int st = 0; st < 16; ++st)
+                    b[t][st] = T == 1 ? (B + (long long)(c * 64 + st) * N)[bo[t]] : B[(long long)(k0 + st) * N + bn[t]];
             }
         }
     };
