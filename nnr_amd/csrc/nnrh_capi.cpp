@@ -448,6 +448,20 @@ extern "C" int nnrh_qconv_dispatch(const nnrh_qconv_desc* d, int* branch) {
 }
 
 namespace {
+// the packed weights of `mats` matrices again behind them, in the small-tile
+// kernel's order
+void append_pieces(std::vector<int8_t>& wp, int mats, int Np, int Kp) {
+    const size_t mat = (size_t)Np * Kp, rows = mat * mats;
+    wp.resize(2 * rows);
+    for (int i = 0; i < mats; ++i) {
+        const int8_t* src = wp.data() + mat * i;
+        int8_t* dst = wp.data() + rows + mat * i;
+        for (int r = 0; r < Np; ++r)
+            for (int k = 0; k < Kp; k += 64)
+                memcpy(dst + piece_off(packed_row_of_col(r), k, Kp), src + (size_t)r * Kp + k, 64);
+    }
+}
+
 // the first layer as one kernel (nnrh_stem.hip): output rows in groups of R
 // (R * oW pixels for the 4 waves' 16-pixel groups), an LDS ring of the rows
 // one group reads plus the next group's, strips of groups per block
@@ -645,13 +659,13 @@ extern "C" int nnrh_qconv_create(nnrh_qconv_t* out, const nnrh_qconv_desc* d) {
             for (int n = 0; n < OCg; ++n) {
                 const int oc = g * OCg + n;
                 const size_t pi = (size_t)g * Np + n;
-                int8_t* const wg = wp.data() + (size_t)g * Np * Kp;
+                int8_t* row = wp.data() + (size_t)g * Np * Kp + packed_off(n, 0, Kp);
                 int32_t s = 0;
                 for (int c = 0; c < Cg; ++c)
                     for (int a = 0; a < d->kH; ++a)
                         for (int b = 0; b < d->kW; ++b) {
                             int8_t v = d->w_host[(((size_t)oc * Cg + c) * d->kH + a) * d->kW + b];
-                            wg[packed_off(n, (a * kWp + b) * Cgp + c, Kp)] = v;
+                            row[(a * kWp + b) * Cgp + c] = v;
                             s += v;
                         }
                 colsum[pi] = s;
@@ -664,6 +678,8 @@ extern "C" int nnrh_qconv_create(nnrh_qconv_t* out, const nnrh_qconv_desc* d) {
                 any_wzp |= betac[pi] != 0;
             }
         for (int32_t v : c0) h->g.c0_absmax = std::max(h->g.c0_absmax, std::llabs((long long)v));
+        const bool small = !first && qgemm_small_size((long long)d->N * sp * OCg * G);
+        if (small) append_pieces(wp, G, Np, Kp);
         if ((rc = upload(&h->wpack, wp.data(), wp.size()))) return fail(rc);
         if ((rc = upload(&h->colsum, colsum.data(), colsum.size()))) return fail(rc);
         if ((rc = upload(&h->c0, c0.data(), c0.size()))) return fail(rc);
@@ -713,6 +729,7 @@ extern "C" int nnrh_qconv_create(nnrh_qconv_t* out, const nnrh_qconv_desc* d) {
             g.lda = h->Cx;
         }
         g.b = h->wpack;
+        g.b_pieces = small ? h->wpack + (size_t)G * Np * Kp : nullptr;
         g.b_bstride = (long long)Np * Kp;
         g.Np = Np;
         g.colsum = h->colsum;
@@ -1154,6 +1171,8 @@ extern "C" int nnrh_qmatmul_create(nnrh_qmatmul_t* out, const nnrh_qmatmul_desc*
     std::vector<int32_t> c0(Np, 0);
     for (int j = 0; j < n; ++j)
         c0[j] = (int32_t)(0u - (uint32_t)(h->a_zp - (au8 ? 128 : 0)) * (uint32_t)colsum[j]);
+    const bool small = qgemm_small_size((long long)d->m * n);
+    if (small) append_pieces(wp, 1, Np, Kp);
     if ((rc = upload(&h->wpack, wp.data(), wp.size()))) return fail(rc);
     if ((rc = upload(&h->colsum, colsum.data(), colsum.size()))) return fail(rc);
     if ((rc = upload(&h->c0, c0.data(), c0.size()))) return fail(rc);
@@ -1182,6 +1201,7 @@ extern "C" int nnrh_qmatmul_create(nnrh_qmatmul_t* out, const nnrh_qmatmul_desc*
     g.M = m; g.N = n; g.K = k; g.Kp = Kp;
     g.lda = k;
     g.b = h->wpack; g.b_bstride = 0; g.Np = Np;
+    g.b_pieces = small ? h->wpack + (size_t)Np * Kp : nullptr;
     g.colsum = h->colsum;
     g.c0 = h->c0;
     g.a_sub = au8 ? 128 : 0;
@@ -1263,6 +1283,8 @@ extern "C" int nnrh_matmul_integer_scaled_create(nnrh_qmatmul_t* out, const nnrh
     std::copy(d->w_scale_host, d->w_scale_host + n, ws.begin());
     if (d->bias_host) std::copy(d->bias_host, d->bias_host + n, b.begin());
     int rc;
+    const bool small = qgemm_small_size((long long)d->m * n);
+    if (small) append_pieces(wp, 1, Np, Kp);
     if ((rc = upload(&h->wpack, wp.data(), wp.size()))) return fail(rc);
     if ((rc = upload(&h->colsum, colsum.data(), colsum.size()))) return fail(rc);
     if ((rc = upload(&h->c0, c0.data(), c0.size()))) return fail(rc);
@@ -1278,6 +1300,7 @@ extern "C" int nnrh_matmul_integer_scaled_create(nnrh_qmatmul_t* out, const nnrh
     g.M = m; g.N = n; g.K = k; g.Kp = Kp;
     g.lda = k;
     g.b = h->wpack; g.b_bstride = 0; g.Np = Np;
+    g.b_pieces = small ? h->wpack + (size_t)Np * Kp : nullptr;
     g.colsum = h->colsum;
     g.c0 = h->c0;
     g.a_sub = au8 ? 128 : 0;
@@ -1343,7 +1366,8 @@ extern "C" int nnrh_qmatmul_group_create(nnrh_qmatmul_group_t* out, const nnrh_q
     const int Np = h0->g.Np, Kp = h0->g.Kp;
     const size_t wsz = (size_t)Np * Kp;
     int rc;
-    if ((rc = nnrh_malloc((void**)&G->wpack, wsz * n))) return fail(rc);
+    const bool small = h0->g.b_pieces != nullptr;   // (of one shape: all members or none)
+    if ((rc = nnrh_malloc((void**)&G->wpack, wsz * n * (small ? 2 : 1)))) return fail(rc);
     if ((rc = nnrh_malloc((void**)&G->colsum, sizeof(int32_t) * Np * n))) return fail(rc);
     if ((rc = nnrh_malloc((void**)&G->c0, sizeof(int32_t) * Np * n))) return fail(rc);
     if ((rc = nnrh_malloc((void**)&G->dq_bias, sizeof(float) * Np * n))) return fail(rc);
@@ -1356,6 +1380,8 @@ extern "C" int nnrh_qmatmul_group_create(nnrh_qmatmul_group_t* out, const nnrh_q
     for (int i = 0; i < n; ++i) {
         const nnrh_qmatmul* h = hs[i];
         if (hipMemcpy(G->wpack + wsz * i, h->wpack, wsz, hipMemcpyDeviceToDevice) != hipSuccess ||
+            (small && hipMemcpy(G->wpack + wsz * (n + i), h->g.b_pieces, wsz, hipMemcpyDeviceToDevice) !=
+                          hipSuccess) ||
             hipMemcpy(G->colsum + (size_t)Np * i, h->colsum, sizeof(int32_t) * Np, hipMemcpyDeviceToDevice) !=
                 hipSuccess ||
             hipMemcpy(G->c0 + (size_t)Np * i, h->c0, sizeof(int32_t) * Np, hipMemcpyDeviceToDevice) != hipSuccess ||
@@ -1373,6 +1399,7 @@ extern "C" int nnrh_qmatmul_group_create(nnrh_qmatmul_group_t* out, const nnrh_q
     }
     g.ngrp = n;
     g.b = G->wpack;
+    g.b_pieces = small ? G->wpack + wsz * n : nullptr;
     g.b_bstride = (long long)wsz;
     g.colsum = G->colsum;
     g.c0 = G->c0;
@@ -1614,7 +1641,7 @@ static int matmul_integer_any(nnrh_matmul_integer* h, const void* a, long long a
     g.a_bstride = a_bstride;
     g.a_xor = au8 ? 0x80 : 0;
     g.M = h->m; g.N = h->n; g.K = h->k; g.Kp = h->Kp;
-    g.b = h->bpack;
+    g.b = g.b_pieces = h->bpack;   // packed below for the one that runs
     g.b_bstride = b_batched ? (long long)h->Np * h->Kp : 0;
     g.Np = h->Np;
     g.param_bstride = b_batched ? h->Np : 0;
@@ -1635,9 +1662,10 @@ static int matmul_integer_any(nnrh_matmul_integer* h, const void* a, long long a
     g.rowsum = g.beta != 0 ? h->rowsum : nullptr;
     g.rowsum_bstride = h->m;
     g.sums_inline = qgemm_small_eligible(g, batch, vec) ? 1 : 0;
+    if (!g.sums_inline) g.b_pieces = nullptr;
     {
         ProfScope ps0("pack_b", s);
-        HIP_TRY(launch_pack_b_dense(b, b_bstride, h->k, h->n, h->Kp, h->Np, bu8 ? 0x80 : 0, h->bpack,
+        HIP_TRY(launch_pack_b_dense(b, b_bstride, h->k, h->n, h->Kp, h->Np, bu8 ? 0x80 : 0, g.sums_inline, h->bpack,
                                     (long long)h->Np * h->Kp, g.sums_inline ? nullptr : h->colsum, h->Np,
                                     b_batched ? batch : 1, s),
                 "pack_b");
@@ -1800,7 +1828,7 @@ struct nnrh_conv_integer {
     int x_dtype = 0, w_dtype = 0, Kp = 0, Np = 0;
     GemmArgs g{};
     uint8_t* xs = nullptr;        // NHWC copy [N][iH][iW][G * Cgp]
-    int8_t* wpack = nullptr;      // [G] x packed_off, Np x Kp bytes each
+    int8_t* wpack = nullptr;      // [G][Np][Kp]
     int32_t* c0 = nullptr;        // [G][Np]
     int32_t* coef = nullptr;      // [G][Np] row-term coefficient
     ~nnrh_conv_integer() {

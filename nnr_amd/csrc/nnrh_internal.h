@@ -45,13 +45,13 @@ struct GemmArgs {
     long long lda;        // dense row stride (bytes)
     long long a_bstride;  // per-batch stride (blockIdx.z)
     int a_xor;            // 0x80 for uint8 activations (x-128), 0 for int8
-    int M, N, K, Kp;      // K real, Kp = K rounded up to 64 (packed B)
+    int M, N, K, Kp;      // K real, Kp = K rounded up to 64 (packed B row length)
     // conv geometry (A_CONV)
     int H, W, C, oH, oW, kH, kW, sH, sW, dH, dW, pad_t, pad_l;
     int Cs;               // channel stride of the NHWC tensor (>= C; groups)
     int kWp;              // > 0: first-layer layout (kW padded to a multiple of 4)
     int pad_byte;         // raw byte for out-of-image taps (x_zp)
-    // ---- B (weights), packed int8 [Np / 16][Kp / 64] 1 KB pieces (packed_off) ----
+    // ---- B (weights), packed [Np][Kp] int8 with the 64-column permutation ----
     const int8_t* b;
     long long b_bstride;
     int Np;
@@ -73,9 +73,6 @@ struct GemmArgs {
     // the Kp bytes of im2col row m (padding reads pad_byte, which must be the
     // zero point alpha + a_sub) taken from the A fragments in the kernel
     const int32_t* row_coef;
-    // small-tile kernel, EPI_I32: it sums A's rows and B's columns itself (colsum
-    // and rowsum unused)
-    int sums_inline;
     // ---- epilogue ----
     int epi;
     int tail;
@@ -145,6 +142,11 @@ struct GemmArgs {
     float add_sa, add_sb, add_fixed;
     int add_a_zp, add_b_zp, add_y_zp;
     long long add_body;
+    // ---- small-tile kernel (last: the other kernels' fields keep their cache
+    // lines of the argument block) ----
+    const int8_t* b_pieces;   // B's bytes in its order (piece_off); NULL: not for it
+    // EPI_I32: it sums A's rows and B's columns itself (colsum and rowsum unused)
+    int sums_inline;
 };
 
 // Multiply-shift constants of an unsigned division by d >= 1 for dividends
@@ -185,6 +187,7 @@ inline long long qgemm_pairs(const GemmArgs& g, int batch) {
 }
 // small-tile kernel for grids that leave the chip idle (nnrh_qgemm_small.hip)
 bool qgemm_small_eligible(const GemmArgs& g, int batch, int vec);
+bool qgemm_small_size(long long outputs);   // false: never for that many
 hipError_t launch_qgemm_small(const GemmArgs& g, int batch, int vec, hipStream_t s);
 // barrier-free short-K kernel (nnrh_qgemm_dma.hip): dense A, Kp = 64, RQ-B
 bool qgemm_direct_eligible(const GemmArgs& g, int batch);
@@ -194,7 +197,7 @@ hipError_t launch_qgemm_direct(const GemmArgs& g, hipStream_t s);
 // NCHW fp32 (or uint8) image with C <= 4 channels -> NHWC uint8, RQ-C.
 struct StemArgs {
     const void* x;          // [N][C][H][W] fp32 or uint8
-    const int8_t* w;        // packed weights (packed_off, 64 columns), K order (kh, kw < 4 * cpr, c < 4)
+    const int8_t* w;        // packed weights [64][Kp], K order (kh, kw < 4 * cpr, c < 4)
     const int32_t* c0;      // [64] accumulator start (-(x_zp - 128) * colsum)
     const float* cs;        // [64] RQ-C scale
     const float* bf;        // [64] RQ-C bias term
@@ -291,30 +294,38 @@ struct ConvIntPrepArgs {
     int copy_blocks, vec;   // set by the launcher
 };
 hipError_t launch_conv_integer_prep(ConvIntPrepArgs a, hipStream_t s);
-// Pack a row-major B[K][N] (int8 or uint8) into the kernels' layout
-// (packed_off) and, unless it is NULL, compute colsum[n] = sum_k (b - b_sub).
+// Pack a row-major B[K][N] (int8 or uint8) into the kernels' layout (packed_off,
+// or piece_off for the small-tile kernel) and, unless it is NULL, compute
+// colsum[n] = sum_k (b - b_sub).
 hipError_t launch_pack_b_dense(const void* b, long long b_bstride, int K,
-                               int N, int Kp, int Np, int b_xor, int8_t* out,
+                               int N, int Kp, int Np, int b_xor, bool pieces, int8_t* out,
                                long long out_bstride, int32_t* colsum,
                                long long colsum_bstride, int batch,
                                hipStream_t s);
 
-// Packed B: offset of byte (column n < Np, k < Kp). A piece is the operand of
-// one MFMA, 16 consecutive columns x 64 K bytes, one contiguous kilobyte (8
-// whole cache lines; as 16 half lines of a row-major [Np][Kp] the same bytes
-// cost the L1 twice as much); the pieces of a column group follow each other
-// along K.
-__host__ __device__ inline long long packed_off(int n, int k, int Kp) {
-    return (long long)(n >> 4) * Kp * 16 + (long long)(k >> 6) * 1024 + (n & 15) * 64 + (k & 63);
-}
-// Row order of a 64-column tile: MFMA row block tn = row / 16 holds columns
-// 16 g + 4 tn + r at rows 4 g + r, so each lane ends with 16 consecutive
-// columns of one output row (see nnrh_qgemm.hip). Its own inverse.
+// Row permutation of packed B inside each 64-column group: storage row of
+// logical column n (its own inverse). The MFMA epilogue then sees 16
+// consecutive columns per lane (see nnrh_qgemm.hip).
 __host__ __device__ inline int packed_row_of_col(int n) {
     int g = n >> 6, nl = n & 63;
     int tn = (nl & 15) >> 2;
     int j = ((nl >> 4) << 2) | (nl & 3);
     return (g << 6) | (tn << 4) | j;
+}
+// Packed B [Np][Kp]: offset of byte (column n < Np, k < Kp).
+__host__ __device__ inline long long packed_off(int n, int k, int Kp) {
+    return (long long)packed_row_of_col(n) * Kp + k;
+}
+// The same for the small-tile kernel, which loads operands straight into
+// registers: a piece is the operand of one MFMA, 16 consecutive columns x 64 K
+// bytes, one contiguous kilobyte, and the pieces of a column group follow each
+// other along K. (It reads the rows above 5 to 20 % slower: 197x3072x768 7.1 ->
+// 8.5 us, conv 8x56x56x64 3x3 7.3 -> 9.1. The kernels that stage tiles in LDS
+// lose as much on pieces: direct 3.6 -> 4.0 us, register-staged 34 -> 42,
+// pipelined 1562x768x1024 7.7 -> 8.0. So weights lie in memory both ways where
+// either kernel may run.)
+__host__ __device__ inline long long piece_off(int n, int k, int Kp) {
+    return (long long)(n >> 4) * Kp * 16 + (long long)(k >> 6) * 1024 + (n & 15) * 64 + (k & 63);
 }
 
 }  // namespace nnrh

@@ -959,14 +959,14 @@ __device__ __forceinline__ void ci_copy(const ConvIntPrepArgs& a, long long i) {
     }
 }
 
-// Pack: one block per column (z, n): its Kp bytes in (kh, kw, c)
+// Pack: one block per packed row (z, n): the row's Kp bytes in (kh, kw, c)
 // order, its column sum, the accumulator start c0 and the row-term coefficient
 __device__ __forceinline__ void ci_pack(const ConvIntPrepArgs& a, int n, int z) {
     __shared__ int32_t part[4];
     const int oc = z * a.OCg + n;
     const int K = a.kH * a.kW * a.Cgp;
     const uint8_t bx = a.w_u8 ? 0x80 : 0;
-    int8_t* const wz = a.wpack + (long long)z * a.Np * a.Kp;
+    int8_t* row = a.wpack + (long long)z * a.Np * a.Kp + packed_off(n, 0, a.Kp);
     int32_t s = 0;
     for (int k = threadIdx.x; k < a.Kp; k += blockDim.x) {
         int8_t v = 0;
@@ -975,7 +975,7 @@ __device__ __forceinline__ void ci_pack(const ConvIntPrepArgs& a, int n, int z) 
             const int kh = t / a.kW, kw = t - kh * a.kW;
             if (c < a.Cg) v = (int8_t)(a.w[(((long long)oc * a.Cg + c) * a.kH + kh) * a.kW + kw] ^ bx);
         }
-        wz[packed_off(n, k, a.Kp)] = v;
+        row[k] = v;
         s += v;
     }
     for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
@@ -1017,15 +1017,15 @@ hipError_t launch_conv_integer_prep(ConvIntPrepArgs a, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------------------
-// Pack a row-major B[K][N] into the GEMM kernels' layout (packed_off), XOR
-// shifting uint8 B to int8, zero padding; colsum[n] = sum_k b'[k][n] by a
-// second kernel. A block turns 64 rows of 64 columns through LDS, so that both
-// the reads (16 bytes of a row a thread) and the writes (whole 1 KB pieces)
-// are contiguous (a thread per 16 k of one column, reading 16 rows, took 4.5
-// us for 96 matrices of 64 x 77).
+// Pack a row-major B[K][N] into the GEMM kernels' layout (packed_off, or
+// piece_off), XOR shifting uint8 B to int8, zero padding; colsum[n] = sum_k
+// b'[k][n] by a second kernel. A block turns 64 rows of 64 columns through LDS,
+// so that the reads (16 bytes of a row a thread) and the writes (64 bytes of a
+// row, or whole 1 KB pieces) are contiguous (a thread per 16 k of one column,
+// reading 16 rows, took 4.5 us for 96 matrices of 64 x 77).
 __global__ __launch_bounds__(256) void pack_b_kernel(const uint8_t* __restrict b,
                                                      long long b_bstride, int K, int N, int Kp,
-                                                     int b_xor, int8_t* __restrict out,
+                                                     int b_xor, int pieces, int8_t* __restrict out,
                                                      long long out_bstride) {
     constexpr int RS = 80;   // LDS row stride: 16-byte stores, rows apart in the banks
     __shared__ __attribute__((aligned(16))) uint8_t tile[64 * RS];
@@ -1058,8 +1058,8 @@ __global__ __launch_bounds__(256) void pack_b_kernel(const uint8_t* __restrict b
         const uint8_t* p = tile + (kc + 4 * q) * RS + c;
         w[q] = p[0] | ((uint32_t)p[RS] << 8) | ((uint32_t)p[2 * RS] << 16) | ((uint32_t)p[3 * RS] << 24);
     }
-    *(uint4*)(out + (long long)blockIdx.y * out_bstride + packed_off(n0 + c, k0 + kc, Kp)) =
-        make_uint4(w[0], w[1], w[2], w[3]);
+    const long long o = pieces ? piece_off(n0 + c, k0 + kc, Kp) : packed_off(n0 + c, k0 + kc, Kp);
+    *(uint4*)(out + (long long)blockIdx.y * out_bstride + o) = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
 __global__ __launch_bounds__(256) void colsum_kernel(const uint8_t* __restrict b,
@@ -1076,12 +1076,12 @@ __global__ __launch_bounds__(256) void colsum_kernel(const uint8_t* __restrict b
 }
 
 hipError_t launch_pack_b_dense(const void* b, long long b_bstride, int K, int N, int Kp, int Np,
-                               int b_xor, int8_t* out, long long out_bstride, int32_t* colsum,
+                               int b_xor, bool pieces, int8_t* out, long long out_bstride, int32_t* colsum,
                                long long colsum_bstride, int batch, hipStream_t s) {
     if (batch <= 0) return hipSuccess;
     dim3 grid((unsigned)((long long)(Np / 64) * (Kp / 64)), batch);
     hipLaunchKernelGGL(pack_b_kernel, grid, dim3(256), 0, s, (const uint8_t*)b, b_bstride, K, N,
-                       Kp, b_xor, out, out_bstride);
+                       Kp, b_xor, pieces ? 1 : 0, out, out_bstride);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (colsum) {

@@ -22,9 +22,9 @@
 // MFMA 16x16 tiles. K advances 64 per step through an LDS double buffer.
 // The MFMA "A" operand is the weight tile (rows = output channels) and the
 // "B" operand the activation tile (columns = output pixels), so lane l holds
-// D[4*(l/16)+r][l%16]. The weights' LDS rows permute the columns inside each
-// 64-column group (packed_row_of_col) so that each lane ends with 16 consecutive
-// output channels of one pixel: one 16-byte store per lane and MFMA tile row.
+// D[4*(l/16)+r][l%16]. Packed weights permute rows inside each 64-column
+// group (packed_row_of_col) so that each lane ends with 16 consecutive output
+// channels of one pixel: one 16-byte store per lane and MFMA tile row.
 #include "nnrh_internal.h"
 #include "nnrh_rq.h"
 
@@ -254,12 +254,12 @@ __global__ __launch_bounds__(256, 2) void qgemm_kernel(GemmArgs g) {
             ra[j].z = (int)(w[2] ^ xmask);
             ra[j].w = (int)(w[3] ^ xmask);
         }
-        // ---- B (packed_off, always in bounds below Np)
+        // ---- B (packed [Np][Kp], always in bounds below Np)
 #pragma unroll
         for (int j = 0; j < B_CH; ++j) {
             int n = ld_n0 + (tid >> 2) + 64 * j;
             if (n < g.Np) {
-                rb[j] = *(const v4i*)(bbase + packed_off(packed_row_of_col(n), k0 + c16 * 16, g.Kp));
+                rb[j] = *(const v4i*)(bbase + (long long)n * g.Kp + k0 + c16 * 16);
             } else {
                 rb[j] = v4i{0, 0, 0, 0};
             }

@@ -293,7 +293,7 @@ void qgemm_dma_kernel(GemmArgs g) {
     const int nk = g.Kp / BK;
     const uint32_t xmask = (uint32_t)g.a_xor * 0x01010101u;
     // KR > 0: this wave's weight fragments of the block's column block, for
-    // every K step of the tile (rows past Np repeat the last column; their
+    // every K step of the tile (rows past Np repeat the last packed row; their
     // outputs are never stored)
     v4i wreg[KR ? KR : 1][4];
     if constexpr (KR > 0) {
@@ -305,7 +305,7 @@ void qgemm_dma_kernel(GemmArgs g) {
             n = n < g.Np ? n : g.Np - 1;
 #pragma unroll
             for (int ks = 0; ks < KR; ++ks)
-                wreg[ks][tn] = *(const v4i*)(g.b + packed_off(packed_row_of_col(n), ks * 64 + fchunk * 16, g.Kp));
+                wreg[ks][tn] = *(const v4i*)(g.b + (long long)n * g.Kp + ks * 64 + fchunk * 16);
         }
     }
     // zero-point column term from the activation zero point (host value or,
@@ -408,14 +408,9 @@ void qgemm_dma_kernel(GemmArgs g) {
         }
 #pragma unroll
         for (int j = 0; j < B_CH; ++j) {
-            // the weights' LDS image is a row of 64 bytes per column for each
-            // MFMA K-step: a wave's DMA then reads 256-byte runs of the packed
-            // pieces (whole lines; 64 bytes of each of two pieces a row, the
-            // image the A rows have, ran 1024x768x3072 2 % slower)
-            const int r = (tid >> 2) + NT / 4 * j, kk = r / BN;
-            int n = p_n0 + r - kk * BN;
+            int n = p_n0 + tid / CPR + RPR * j;
             n = n < g.Np ? n : g.Np - 1;
-            b_addr[j] = (uint64_t)(pb + packed_off(packed_row_of_col(n), kk * 64 + ((tid & 3) ^ dma_swz<64>(r)) * 16, g.Kp));
+            b_addr[j] = (uint64_t)(pb + (long long)n * g.Kp + cdma * 16);
         }
         if constexpr (AMODE == A_CONV) {
             const int k = cdma * 16;
@@ -462,7 +457,7 @@ void qgemm_dma_kernel(GemmArgs g) {
         if constexpr (KR == 0) {
 #pragma unroll
             for (int j = 0; j < B_CH; ++j)
-                dma16((const void*)(b_addr[j] + (uint64_t)k0 * 16), st + BM * BK + wave * 1024 + j * RND);
+                dma16((const void*)(b_addr[j] + (uint64_t)k0), st + BM * BK + wave * 1024 + j * RND);
         }
         if (p_kt == 0 && wave < PWAVES) {
             // per-column constants of the tile: NP arrays of BN int32/float,
@@ -953,7 +948,7 @@ void qgemm_dma_kernel(GemmArgs g) {
         } else {
 #pragma unroll
             for (int tn = 0; tn < 4; ++tn)
-                wf[tn] = *(const v4i*)(st + BM * BK + kk * BN * 64 + dma_lds_off<64>(wn * 64 + tn * 16 + frow, fchunk));
+                wf[tn] = *(const v4i*)(st + BM * BK + dma_lds_off<BK>(wn * 64 + tn * 16 + frow, c));
         }
     };
     auto mma = [&](const v4i (&xf)[4], const v4i (&wf)[4], bool first) {
@@ -1124,8 +1119,7 @@ __global__ __launch_bounds__(256, 2) void qgemm_direct_kernel(GemmArgs g) {
         int n = cb * 64 + tn * 16 + frow;
         n = n < g.Np ? n : g.Np - 1;
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
-            wreg[ks][tn] = *(const v4i*)(g.b + packed_off(packed_row_of_col(n), ks * 64 + fchunk * 16, g.Kp));
+        for (int ks = 0; ks < KS; ++ks) wreg[ks][tn] = *(const v4i*)(g.b + (long long)n * g.Kp + ks * 64 + fchunk * 16);
         c0v[tn] = *(const v4i*)(g.c0 + nb + 4 * tn);
         const v4i o = *(const v4i*)(g.os + nb + 4 * tn);
 #pragma unroll

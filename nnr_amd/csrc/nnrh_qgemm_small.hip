@@ -132,7 +132,7 @@ __global__ __launch_bounds__(MAXW * 64) void qgemm_small_kernel(SmallArgs s, Gem
     const int8_t* b_row[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
-        b_row[nt] = bbase + packed_off(n0 + 16 * nt + frow, fchunk * 16, s.Kp);
+        b_row[nt] = bbase + piece_off(n0 + 16 * nt + frow, fchunk * 16, s.Kp);
 
     // ---- K loop
     auto load_a = [&](int k, v4i (&xf)[MT]) {
@@ -587,7 +587,7 @@ template <int MT, int NT, int AMODE, int VEC, int EP, int MAXW>
 hipError_t launch_small(const GemmArgs& g, int batch, int W, hipStream_t st) {
     constexpr int BM = 16 * MT, BN = 16 * NT;
     SmallArgs s{};
-    s.a = g.a; s.b = g.b; s.a_bstride = g.a_bstride; s.b_bstride = g.b_bstride;
+    s.a = g.a; s.b = g.b_pieces; s.a_bstride = g.a_bstride; s.b_bstride = g.b_bstride;
     s.M = g.M; s.N = g.N; s.K = g.K; s.Kp = g.Kp;
     s.nbm = (g.M + BM - 1) / BM;
     s.nbn = (g.N + BN - 1) / BN;
@@ -687,13 +687,15 @@ constexpr long long SMALL_MAX_OUT = 1650000, SMALL_MAX_OUT_REG = 3300000;
 
 // (a fused epilogue is refused where the pipelined kernel refuses it)
 static bool small_modes(const GemmArgs& g, int batch, bool pipelined) {
-    if (g.kWp > 0 || g.row_coef || g.epi == EPI_RQC || g.tail == TAIL_OW) return false;
+    if (!g.b_pieces || g.kWp > 0 || g.row_coef || g.epi == EPI_RQC || g.tail == TAIL_OW) return false;
     if (g.epi == EPI_I32 ? !g.sums_inline || g.H > 0 : g.c0 == nullptr && g.colsum == nullptr) return false;
     if ((g.add_other || g.dq_bias) && !pipelined) return false;
     if (batch > 65535 || g.lda > 0x7fffffffLL) return false;
     const long long out = (long long)g.M * g.N * batch;
     return out <= (pipelined ? SMALL_MAX_OUT : SMALL_MAX_OUT_REG);
 }
+
+bool qgemm_small_size(long long outputs) { return outputs <= SMALL_MAX_OUT_REG; }
 
 bool qgemm_small_eligible(const GemmArgs& g, int batch, int vec) {
     return small_modes(g, batch, qgemm_dma_eligible(g, vec) || qgemm_direct_eligible(g, batch));

@@ -135,8 +135,8 @@ __global__ __launch_bounds__(256, 2) void stem_conv_kernel(StemArgs a) {
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
         for (int tn = 0; tn < NT; ++tn) {
-            const int col = (frow >> 2) * 4 * NT + 4 * tn + (frow & 3);
-            wf[ks][tn] = *(const v4i*)(a.w + packed_off(col, ks * 64 + fch * 16, a.Kp));
+            const int row = packed_row_of_col((frow >> 2) * 4 * NT + 4 * tn + (frow & 3));
+            wf[ks][tn] = *(const v4i*)(a.w + (long long)row * a.Kp + ks * 64 + fch * 16);
         }
     // per-column constants of this lane's 4 NT columns
     v4i c0v[NT], csv[NT], bfv[NT];
