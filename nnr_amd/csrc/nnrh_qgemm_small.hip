@@ -674,14 +674,51 @@ hipError_t launch_small_tile(const GemmArgs& g, int batch, hipStream_t s) {
     }
 }
 
-// outputs up to which this kernel is the faster one (measured on dense and 3x3
-// shapes of N = 64 .. 1024, K = 64 .. 4608). Against the pipelined kernel:
-// 12544x128x128 4.1 / 4.8 us, 1024x768x3072 12.0 / 19.7, 2048x768x3072 16.2 /
-// 20.1, conv 12544x128x1152 10.1 / 11.4, level at 1.6 M outputs (6272x256x2304
-// 16.6 / 17.0) and behind at twice that (12544x256x512 10.2 / 7.2). Against
-// the register-staged one, at NCHW output: conv 1568x64x576 4.7 / 29.7,
-// 50176x64x576 19.8 / 30.7, 12544x256x256 13.1 / 18.8, level at 6.4 M.
-constexpr long long SMALL_MAX_OUT = 1650000, SMALL_MAX_OUT_REG = 3300000;
+// Outputs up to which this kernel is the faster one, as its time over the other
+// kernel's at thousands of outputs (graphs of calls whose operands come from the
+// Infinity Cache, as a layer's do; N = 16 .. 3072, 7 .. 56 pixels). Against the
+// register-staged kernel at any K up to 3.3 M: NCHW 3x3 0.34 at 1000, 0.67 at
+// 3250, K % 16 != 0 0.35, 0.5; with a weight zero point 0.90 at 2800, 1.04 at 3250.
+constexpr long long SMALL_MAX_OUT_REG = 3300000, SMALL_MAX_OUT_ROWSUM = 2800000;
+
+// Against the pipelined and direct kernels:
+long long small_max_out(const GemmArgs& g, int batch) {
+    const int K = g.Kp;
+    if (g.epi == EPI_I32) return 1650000;   // 0.77 at 1600 with its pass over B
+    if (g.mm_parts) {
+        // the (min, max) pairs allow few tiles smaller than 64 x 64. With Gelu K =
+        // 64 and 128 1.25 at any size; 192 0.80 and 256 0.85 to 1600, 1.45 at 2200;
+        // 768 0.53 at 1000, 0.95 at 1600, 1.3 at 2200. Without, the epilogue does
+        // not cover a second round of blocks on the 256 CUs: K = 512 and more 0.70
+        // up to one, 1.2 past it (3072 0.94); 320 and 384 0.95, 1.04; 192 and 256 1.0
+        // +- 0.1
+        if (g.dq_gelu) return K < 192 ? 0 : 1650000;
+        return K < 320 ? 0 : K < 2048 ? 256 * 64 * 64 : 1650000;
+    }
+    if (g.dq_bias) return 1650000;   // fp32 chains 0.85 at 1600, K = 32 .. 3072
+    // convolution groups of 64 channels, 3x3 0.67 at 1000, 1.02 at 1250; 1x1 of
+    // K = 128 0.87 at 600, 1.16 at 800; of 32 0.92 at 1250, 1.2 at 1600; of 16
+    // 0.84 at 1600
+    if (batch > 1 && g.oH > 0) return g.N <= 16 ? 1650000 : g.N <= 32 ? 1300000 : K < 256 ? 700000 : 1220000;
+    if (g.epi == EPI_RQD) {
+        if (g.N < 64) return K <= 64 ? 1350000 : 1650000;   // 0.95 at 1250, 1.02 at 1600; 256 0.8
+        // K = 64 0.96 at 600, 1.12 at 800; 128 0.93 at 800, 1.07 at 1000; 256 0.95
+        // at 1000, 1.0 at 1250; 320 and 384 (three units of K on two waves) 0.86
+        // at 600, 1.02 at 800; 512 .. 3072 0.92 at 1250, 1.10 at 1600
+        return K <= 64 ? 650000 : K <= 128 ? 850000 : K <= 256 ? 1200000 : K <= 384 ? 750000 : 1350000;
+    }
+    if (g.add_other) {
+        // K = 64 0.97 at 800, 1.05 at 1200, but 0.76 at 1600 where theirs holds the
+        // weights in registers; 128 0.92 at 800, 1.0 at 1200; 192 and 256 0.82 at
+        // 1250, 1.0 at 1600; 320 and 384 0.93 at 1000, 1.0 at 1250; 512 .. 2048 0.90
+        // at 1600
+        if (K == 64 && g.N > 64 && g.M > 128 * 31) return 1650000;
+        return K <= 64 ? 1000000 : K <= 128 ? 1250000 : K <= 256 ? 1500000 : K < 512 ? 1250000 : 1650000;
+    }
+    // K = 64 0.95 at 1200, 1.0 .. 1.1 at 1600 (16 channels 0.9); 128 0.74, 256 0.86,
+    // 1152 0.92 at 1600; 2048, 2304 and 4608 0.92 at 1250, 1.03 at 1600
+    return K <= 64 ? (g.N <= 16 ? 1650000 : 1200000) : K < 2048 ? 1650000 : 1450000;
+}
 
 }  // namespace
 
@@ -691,8 +728,13 @@ static bool small_modes(const GemmArgs& g, int batch, bool pipelined) {
     if (g.epi == EPI_I32 ? !g.sums_inline || g.H > 0 : g.c0 == nullptr && g.colsum == nullptr) return false;
     if ((g.add_other || g.dq_bias) && !pipelined) return false;
     if (batch > 65535 || g.lda > 0x7fffffffLL) return false;
-    const long long out = (long long)g.M * g.N * batch;
-    return out <= (pipelined ? SMALL_MAX_OUT : SMALL_MAX_OUT_REG);
+    if (!pipelined)
+        return (long long)g.M * g.N * batch <=
+               (g.rowsum && g.epi != EPI_I32 ? SMALL_MAX_OUT_ROWSUM : SMALL_MAX_OUT_REG);
+    // (a count of 64 x 64 blocks decides there)
+    const bool blocks = g.mm_parts && !g.dq_gelu;
+    const long long m = blocks ? (g.M + 63) & ~63 : g.M, n = blocks ? (g.N + 63) & ~63 : g.N;
+    return m * n * batch <= small_max_out(g, batch);
 }
 
 bool qgemm_small_size(long long outputs) { return outputs <= SMALL_MAX_OUT_REG; }

@@ -42,6 +42,7 @@ def variants(run):
 
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (15, 17, 16), (16, 16, 64), (17, 33, 65), (1, 3072, 768), (31, 4, 128),
                                    (33, 130, 192), (49, 512, 4608), (96, 96, 72), (61, 8, 24), (3, 1000, 2041),
+                                   (634, 1024, 48), (635, 1024, 48), (1318, 1024, 512), (1319, 1024, 512),
                                    (1611, 1024, 48), (1612, 1024, 48), (3222, 1024, 20), (3223, 1024, 20)])
 @pytest.mark.parametrize("dt", [np.uint8, np.int8])
 def test_matmul(dev, m, n, k, dt):
@@ -52,8 +53,10 @@ def test_matmul(dev, m, n, k, dt):
     op = H.QLinearMatMul(b, *args[:2], *args[3:], m=m, a_dtype=dt, y_dtype=dt)
     y, names = variants(lambda: op(on(dev, a)))
     assert np.array_equal(y.reshape(ref.shape), ref)
-    # the pipelined kernel takes K % 16 == 0, the register-staged one the rest
-    limit = 1650000 if k % 16 == 0 else 3300000
+    # the pipelined kernel takes K % 16 == 0, the register-staged one the rest.
+    # (One limit of 1650000 for every K had the small-tile kernel run K = 64 at
+    # 800000 outputs and more, 1.1 to 1.27 times the pipelined kernel's time)
+    limit = 3300000 if k % 16 else 650000 if k <= 64 else 1350000
     assert any("small" in v for v in names) == (m * n <= limit), names
 
 
