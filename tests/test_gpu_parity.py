@@ -1156,7 +1156,8 @@ def test_global_avgpool_dequant(dev, nhwc, dt, C):
 
 
 @pytest.mark.parametrize("N,C,HW", [(1, 3, 1), (2, 65, 31), (1, 2048, 32), (3, 70, 33), (1, 64, 65),   # one channel a thread
-                                    (32, 2048, 49), (33, 2048, 49), (33, 2050, 33)])   # its last size; past it
+                                    (32, 2048, 49), (33, 2048, 49), (33, 2050, 33),   # its last size; past it
+                                    (2, 64, 3), (2, 65, 3), (2, 64, 4)])   # too few pixels for it; enough
 @pytest.mark.parametrize("dt", [np.uint8, np.int8])
 def test_global_avgpool_dequant_sizes(dev, N, C, HW, dt):
     """NHWC at the edges of the 32-pixel steps and of the output count up to
