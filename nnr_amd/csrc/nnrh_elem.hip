@@ -514,10 +514,12 @@ __global__ __launch_bounds__(256) void dynq_codes_direct_kernel(const uint8_t* _
         if (j < nc) y[o + j] = (uint8_t)(w >> (8 * j));
 }
 
-// rows up to which every element takes the expression itself (3072 columns with
-// Gelu; table + gather / direct): 37 rows 11.3 / 3.4 us,
-// 256 14.3 / 4.3, 512 14.3 / 5.7, 1024 14.3 / 9.3
-constexpr long long DQC_DIRECT_ROWS = 1024;
+// Rows and elements up to which every element takes the expression itself (with
+// Gelu, table + gather / direct): 3072 columns 37 rows 11.3 / 3.4 us, 256 14.3 /
+// 4.3, 1024 14.3 / 9.3; 8192 columns 768 rows 17.4 / 17.0, 1024 18.9 / 19.5; 16384
+// columns 384 rows 22.5 / 17.2, 640 22.9 / 25.7, 1024 24.3 / 42.1. (More rows of
+// fewer columns were not measured.)
+constexpr long long DQC_DIRECT_ROWS = 1024, DQC_DIRECT_MAX = 768 * 8192;
 
 size_t dynamic_quantize_codes_table_bytes(int Np) { return (size_t)256 * (size_t)Np; }
 
@@ -525,7 +527,7 @@ hipError_t launch_dynamic_quantize_codes(const uint8_t* codes, long long rows, i
                                          float dq_scale, int q_zp, int gelu, const float* parts, int nparts,
                                          uint8_t* table, uint8_t* y, float* y_scale, uint8_t* y_zp,
                                          hipStream_t s) {
-    if (rows > 0 && rows <= DQC_DIRECT_ROWS) {
+    if (rows > 0 && rows <= DQC_DIRECT_ROWS && rows * N <= DQC_DIRECT_MAX) {
         hipLaunchKernelGGL(dynq_codes_direct_kernel, dim3((unsigned)((N + 1023) / 1024), (unsigned)rows), dim3(256), 0,
                            s, codes, N, parts, nparts, bias, dq_scale, q_zp, gelu, y, y_scale, y_zp);
         return hipGetLastError();

@@ -694,9 +694,11 @@ def test_qmatmul_fused_gelu_minmax(dev, m, n, batch):
 
 @pytest.mark.parametrize("m,n,batch,gelu", [(40, 136, 3, True), (8192 // 64, 3072, 2, True), (70, 64, 1, False),
                                              (50, 320, 2, True), (33, 200, 2, False), (21, 131, 2, True),
-                                             # one element a thread up to 1024 rows; the table past it
+                                             # every element by itself (4 a thread) up to 1024 rows and
+                                             # 768 x 8192 elements; the table past either
                                              (1, 1, 1, True), (1, 1027, 1, False), (512, 1028, 2, True),
-                                             (1025, 131, 1, True), (1025, 1028, 1, True)])
+                                             (1025, 131, 1, True), (1025, 1028, 1, True),
+                                             (768, 8192, 1, False), (769, 8192, 1, True)])
 def test_qmatmul_codes_dynamic_quantize(dev, m, n, batch, gelu):
     """The fused QLinearMatMul -> DequantizeLinear -> + bias (-> Gelu) chain
     in codes mode: a run stores the uint8 QLinearMatMul bytes (equal to the
