@@ -1044,10 +1044,14 @@ __global__ __launch_bounds__(256, 3) void mha_fused_hd64_kernel(const float* __r
 // The products use the operand orders of the kernel above: scores as S^T (lane
 // (g, lr) holds keys 16 tt + 4 g + i of query lr), which is the A operand of P
 // V; a lane of O holds queries 4 g + i.
+// wscale, a power of two of at most 1 / S, keeps the sums of weights times values
+// within the values' range (S weights of 1 and values of 2^127 would overflow
+// before the division by the sum of weights). It changes no bit of the rest and
+// costs up to 3 % (32 heads x 512 x 32 21.8 -> 22.5 us).
 template <int HD>
 __global__ __launch_bounds__(256, HD <= 64 ? 4 : HD <= 96 ? 3 : 2) void mha_flash_kernel(
     const float* __restrict q, const float* __restrict k, const float* __restrict v, float* __restrict y, int S,
-    int Hd, int nh, int nqb, int total, float scale) {
+    int Hd, int nh, int nqb, int total, float scale, float wscale) {
     constexpr int KB = 64;                 // keys a step
     constexpr int RS = HD + 4;             // LDS row stride (floats): 16 rows apart in the banks
     constexpr int H4 = HD / 4;             // floats of a row one lane group multiplies
@@ -1143,7 +1147,7 @@ __global__ __launch_bounds__(256, HD <= 64 ? 4 : HD <= 96 ? 3 : 2) void mha_flas
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float e = expf(p[tt][i] - mu);
-                p[tt][i] = e;
+                p[tt][i] = e * wscale;
                 sum += e;
             }
         sum += __shfl_xor(sum, 16, 64);
@@ -1180,7 +1184,7 @@ __global__ __launch_bounds__(256, HD <= 64 ? 4 : HD <= 96 ? 3 : 2) void mha_flas
             stage();
         }
     }
-    const float inv = 1.0f / l;
+    const float inv = 1.0f / (l * wscale);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const float a = __shfl(inv, 4 * g + i, 64);
@@ -1212,11 +1216,13 @@ static bool launch_mha_flash(const float* q, const float* k, const float* v, flo
     auto over = [&](const float* x) { return y < x + n && x < y + n; };
     if (over(k) || (over(q) && y != q)) return false;
     const dim3 grid((unsigned)(8 * ((total + 7) / 8)));
+    float wscale = 1.0f;
+    while (wscale * (float)S > 1.0f) wscale *= 0.5f;
     switch (Hd / nh) {
 #define NNRH_FLASH_CASE(HD)                                                                                        \
     case HD:                                                                                                       \
         hipLaunchKernelGGL(mha_flash_kernel<HD>, grid, dim3(256), 0, s, q, k, v, y, S, Hd, nh, nqb, (int)total, \
-                           scale);                                                                                 \
+                           scale, wscale);                                                                                 \
         return true;
         NNRH_FLASH_CASE(32) NNRH_FLASH_CASE(64) NNRH_FLASH_CASE(80) NNRH_FLASH_CASE(96) NNRH_FLASH_CASE(128)
 #undef NNRH_FLASH_CASE

@@ -58,6 +58,19 @@ def test_large_scores(dev):
     assert np.linalg.norm(y - ref) <= 1e-3 * np.linalg.norm(ref)
 
 
+@pytest.mark.parametrize("hd,S", [(64, 129), (64, 512), (32, 300), (128, 1000)])
+def test_large_values(dev, hd, S):
+    """Values whose sum over the keys is no float, whose weighted mean is one."""
+    q, k, v = data(6 + S, 1, S, hd)
+    v = np.sign(v) * np.random.default_rng(S).uniform(2e38, 3e38, v.shape).astype(np.float32)
+    v[..., 0] = 3e38   # a column of equal values: nothing cancels
+    q *= np.float32(0.1)
+    y, ref = attention(dev, q, k, v, 1, 0.125), exact(q, k, v, 1, 0.125)
+    assert np.isfinite(y).all()
+    # (scaled: the squares of the norm are no floats; the bound of ordinary values)
+    assert np.linalg.norm(y / 1e38 - ref / 1e38) <= 1.2e-6 * np.linalg.norm(ref / 1e38)
+
+
 def test_infinite_scores(dev):
     """Keys whose scores are -inf weigh nothing, a whole step of them too (the
     first 64 keys); a row with only such keys, or with +inf, is NaN."""
