@@ -473,10 +473,14 @@ int nnrh_global_avgpool_f32(const float* x_dev, float* y_dev, int N, int C, int 
  * head_dim; y = softmax(scale * Q_h K_h^T) V_h per (batch, head), with the
  * heads read and written in place. Head size 64 with seq <= 128 (and q, k,
  * v, y 16-byte aligned) runs as one fused fp32-MFMA kernel per (batch,
- * head) and needs no workspace (NULL is accepted); other shapes use batched
- * GEMMs and a scaled softmax over a workspace of at least
- * nnrh_multihead_attention_workspace bytes, 256-byte aligned. The size is 0
- * for the fused shapes. minmax_parts (optional, NULL for none; no
+ * head) and needs no workspace (NULL is accepted). Other shapes are given a
+ * workspace of at least nnrh_multihead_attention_workspace bytes (the score
+ * matrix; 0 for the fused shapes), 256-byte aligned. Head sizes 32, 64, 80,
+ * 96 and 128, 16-byte aligned, run as one kernel that walks the keys and
+ * leaves it untouched, unless y lies over k or, other than exactly, over q;
+ * the rest as batched GEMMs and a scaled softmax over it. y over v is refused
+ * (NNRH_ERR_INVALID) outside the fused kernel, except exactly over v with seq
+ * <= 64. minmax_parts (optional, NULL for none; no
  * counterpart in the reference): the fused kernel also writes (min, max)
  * pairs of y for a DynamicQuantizeLinear that reads it
  * (nnrh_dynamic_quantize_linear_parts), nnrh_multihead_attention_minmax_count

@@ -2072,6 +2072,11 @@ extern "C" int nnrh_multihead_attention_f32(const float* q, const float* k, cons
                                                         "seq <= 128, 16-byte aligned q / k / v / y)"
                                                       : "mha: this shape (or unaligned q / k / v / y) needs the workspace");
     if (((uintptr_t)workspace & 255) != 0) return set_err(NNRH_ERR_INVALID, "mha: workspace must be 256-byte aligned");
+    // outside the fused kernel a head's queries are split over blocks of 64 that
+    // all read its values to the end: what one has written another would read
+    const size_t n = (size_t)B * seq * hidden;
+    if (!mha_fused_ok(q, k, v, y, seq, hidden, num_heads) && y < v + n && v < y + n && !(y == v && seq <= 64))
+        return set_err(NNRH_ERR_INVALID, "mha: y lies over v");
     hipStream_t s = S(stream);
     ProfScope ps("multihead_attention", s);
     HIP_TRY(launch_mha_f32(q, k, v, y, B, seq, hidden, num_heads, scale, minmax_parts, workspace, s),

@@ -111,3 +111,14 @@ def test_group_create_errors():
     assert b"no contexts" in L.nnr_last_error()
     assert g.value is None
     assert L.nnr_group_destroy(None) == 0
+
+
+@pytest.mark.parametrize("seq,off", [(65, 0), (129, 0), (129, 256), (129, -256), (64, 256), (200, 199 * 768 * 4)])
+@pytest.mark.parametrize("hd", [32, 48])   # one kernel over the keys; GEMMs and softmax
+def test_attention_output_over_values_is_refused(seq, off, hd):
+    """Blocks of one head's queries all read its values: an output there is an
+    error before anything launches (the addresses are no memory)."""
+    L, heads = _lib.lib(), 768 // hd
+    q, k, v, ws = (0x10000000 * (i + 1) for i in range(4))
+    rc = L.nnrh_multihead_attention_f32(q, k, v, v + off, 1, seq, 768, heads, 0.1, None, ws, None)
+    assert rc == _lib.NNRH_ERR_INVALID and "over v" in L.nnrh_last_error().decode()

@@ -87,8 +87,9 @@ def test_infinite_scores(dev):
     assert np.isnan(y[0, 7]).all() and not np.isnan(np.delete(y[0], 7, 0)).any()
 
 
-@pytest.mark.parametrize("over", ["q", "k"])
-def test_output_over_an_input(dev, over):
-    q, k, v = data(5, 2, 260, 128)
+@pytest.mark.parametrize("over,S,hd", [("q", 260, 64), ("k", 260, 64),
+                                       ("v", 64, 32), ("v", 64, 48), ("v", 64, 128)])   # one block a head
+def test_output_over_an_input(dev, over, S, hd):
+    q, k, v = data(5, 2, S, 2 * hd)
     y, ref = attention(dev, q, k, v, 2, 0.125, over), exact(q, k, v, 2, 0.125)
     assert np.linalg.norm(y - ref) <= 1.2e-6 * np.linalg.norm(ref)
