@@ -12,6 +12,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <new>
 #include <string>
 #include <vector>
@@ -462,6 +463,31 @@ void append_pieces(std::vector<int8_t>& wp, int mats, int Np, int Kp) {
     }
 }
 
+// a row-major B [k][n], XOR x, as packed rows and, with `small`, as pieces behind
+// them, and its column sums; 64 x 64 bytes at a time, so that a column's reads
+// stay in the L1, and each column's 64 bytes to both places at once
+std::unique_ptr<int8_t[]> pack_dense(const uint8_t* b, int k, int n, uint8_t x, int Kp, int Np, bool small,
+                                     std::vector<int32_t>& colsum) {
+    const size_t mat = (size_t)Np * Kp;
+    std::unique_ptr<int8_t[]> wp(new int8_t[mat * (small ? 2 : 1)]);
+    for (int j0 = 0; j0 < Np; j0 += 64)
+        for (int i0 = 0; i0 < Kp; i0 += 64)
+            for (int j = j0; j < j0 + 64; ++j) {
+                int8_t v[64];
+                int32_t s = 0;
+                const int rows = j < n ? std::min(k - i0, 64) : 0;
+                if (rows == 64)
+                    for (int i = 0; i < 64; ++i) v[i] = (int8_t)(b[(size_t)(i0 + i) * n + j] ^ x);
+                else
+                    for (int i = 0; i < 64; ++i) v[i] = i < rows ? (int8_t)(b[(size_t)(i0 + i) * n + j] ^ x) : 0;
+                for (int i = 0; i < 64; ++i) s += v[i];
+                colsum[j] += s;
+                memcpy(wp.get() + packed_off(j, i0, Kp), v, 64);
+                if (small) memcpy(wp.get() + mat + piece_off(j, i0, Kp), v, 64);
+            }
+    return wp;
+}
+
 // the first layer as one kernel (nnrh_stem.hip): output rows in groups of R
 // (R * oW pixels for the 4 waves' 16-pixel groups), an LDS ring of the rows
 // one group reads plus the next group's, strips of groups per block
@@ -650,7 +676,10 @@ extern "C" int nnrh_qconv_create(nnrh_qconv_t* out, const nnrh_qconv_desc* d) {
         const int a_sub = u8 ? 128 : 0;
         const int alpha = d->x_zp - a_sub;
         const bool rqb = br == NNRH_BR_PACKED || br == NNRH_BR_NR16;
-        std::vector<int8_t> wp((size_t)G * Np * Kp, 0);
+        const bool small = !first && qgemm_small_size((long long)d->N * sp * OCg * G);
+        std::vector<int8_t> wp;
+        wp.reserve((size_t)G * Np * Kp * (small ? 2 : 1));
+        wp.resize((size_t)G * Np * Kp, 0);
         std::vector<int32_t> colsum((size_t)G * Np, 0), c0((size_t)G * Np, 0), biasp((size_t)G * Np, 0),
             betac((size_t)G * Np, 0);
         std::vector<float> osp((size_t)G * Np, 0.f), csp((size_t)G * Np, 0.f), bfp((size_t)G * Np, 0.f);
@@ -661,13 +690,17 @@ extern "C" int nnrh_qconv_create(nnrh_qconv_t* out, const nnrh_qconv_desc* d) {
                 const size_t pi = (size_t)g * Np + n;
                 int8_t* row = wp.data() + (size_t)g * Np * Kp + packed_off(n, 0, Kp);
                 int32_t s = 0;
-                for (int c = 0; c < Cg; ++c)
-                    for (int a = 0; a < d->kH; ++a)
-                        for (int b = 0; b < d->kW; ++b) {
-                            int8_t v = d->w_host[(((size_t)oc * Cg + c) * d->kH + a) * d->kW + b];
-                            row[(a * kWp + b) * Cgp + c] = v;
+                const int taps = d->kH * d->kW;
+                const int8_t* src = d->w_host + (size_t)oc * Cg * taps;
+                for (int a = 0; a < d->kH; ++a)
+                    for (int b = 0; b < d->kW; ++b) {
+                        int8_t* dst = row + (a * kWp + b) * Cgp;
+                        for (int c = 0; c < Cg; ++c) {
+                            const int8_t v = src[(size_t)c * taps + a * d->kW + b];
+                            dst[c] = v;
                             s += v;
                         }
+                    }
                 colsum[pi] = s;
                 biasp[pi] = bias[oc];
                 // c0 = (RQ-B: bias) - alpha * colsum, int32 wrap-around
@@ -678,7 +711,6 @@ extern "C" int nnrh_qconv_create(nnrh_qconv_t* out, const nnrh_qconv_desc* d) {
                 any_wzp |= betac[pi] != 0;
             }
         for (int32_t v : c0) h->g.c0_absmax = std::max(h->g.c0_absmax, std::llabs((long long)v));
-        const bool small = !first && qgemm_small_size((long long)d->N * sp * OCg * G);
         if (small) append_pieces(wp, G, Np, Kp);
         if ((rc = upload(&h->wpack, wp.data(), wp.size()))) return fail(rc);
         if ((rc = upload(&h->colsum, colsum.data(), colsum.size()))) return fail(rc);
@@ -1153,27 +1185,16 @@ extern "C" int nnrh_qmatmul_create(nnrh_qmatmul_t* out, const nnrh_qmatmul_desc*
     const int m = d->m, n = d->n, k = d->k;
     const int Kp = round_up(k, 64), Np = round_up(n, 64);
     const bool bu8 = d->b_dtype == NNRH_U8;
-    std::vector<int8_t> wp((size_t)Np * Kp, 0);
+    const bool small = qgemm_small_size((long long)m * n);
     std::vector<int32_t> colsum(Np, 0);
-    const uint8_t* braw = (const uint8_t*)d->b_host;
-    for (int j = 0; j < n; ++j) {
-        int32_t s = 0;
-        for (int i = 0; i < k; ++i) {
-            int8_t v = (int8_t)(braw[(size_t)i * n + j] ^ (bu8 ? 0x80 : 0));
-            wp[packed_off(j, i, Kp)] = v;
-            s += v;
-        }
-        colsum[j] = s;
-    }
+    const auto wp = pack_dense((const uint8_t*)d->b_host, k, n, bu8 ? 0x80 : 0, Kp, Np, small, colsum);
     int rc;
     const bool au8 = d->a_dtype == NNRH_U8;
     h->a_zp = ld_zp(d->a_zp_host, d->a_dtype);
     std::vector<int32_t> c0(Np, 0);
     for (int j = 0; j < n; ++j)
         c0[j] = (int32_t)(0u - (uint32_t)(h->a_zp - (au8 ? 128 : 0)) * (uint32_t)colsum[j]);
-    const bool small = qgemm_small_size((long long)d->m * n);
-    if (small) append_pieces(wp, 1, Np, Kp);
-    if ((rc = upload(&h->wpack, wp.data(), wp.size()))) return fail(rc);
+    if ((rc = upload(&h->wpack, wp.get(), (size_t)Np * Kp * (small ? 2 : 1)))) return fail(rc);
     if ((rc = upload(&h->colsum, colsum.data(), colsum.size()))) return fail(rc);
     if ((rc = upload(&h->c0, c0.data(), c0.size()))) return fail(rc);
     for (int32_t v : c0) h->g.c0_absmax = std::max(h->g.c0_absmax, std::llabs((long long)v));
@@ -1263,18 +1284,9 @@ extern "C" int nnrh_matmul_integer_scaled_create(nnrh_qmatmul_t* out, const nnrh
     auto fail = [&](int code) { delete h; return code; };
     const int m = d->m, n = d->n, k = d->k;
     const int Kp = round_up(k, 64), Np = round_up(n, 64);
-    std::vector<int8_t> wp((size_t)Np * Kp, 0);
+    const bool small = qgemm_small_size((long long)m * n);
     std::vector<int32_t> colsum(Np, 0);
-    const uint8_t* braw = (const uint8_t*)d->b_host;
-    for (int j = 0; j < n; ++j) {
-        int32_t sum = 0;
-        for (int i = 0; i < k; ++i) {
-            const int8_t v = (int8_t)(braw[(size_t)i * n + j] ^ (bu8 ? 0x80 : 0));
-            wp[packed_off(j, i, Kp)] = v;
-            sum += v;
-        }
-        colsum[j] = sum;
-    }
+    const auto wp = pack_dense((const uint8_t*)d->b_host, k, n, bu8 ? 0x80 : 0, Kp, Np, small, colsum);
     const bool au8 = d->a_dtype == NNRH_U8;
     std::vector<int32_t> c0(Np, 0);
     for (int j = 0; j < n; ++j)
@@ -1283,9 +1295,7 @@ extern "C" int nnrh_matmul_integer_scaled_create(nnrh_qmatmul_t* out, const nnrh
     std::copy(d->w_scale_host, d->w_scale_host + n, ws.begin());
     if (d->bias_host) std::copy(d->bias_host, d->bias_host + n, b.begin());
     int rc;
-    const bool small = qgemm_small_size((long long)d->m * n);
-    if (small) append_pieces(wp, 1, Np, Kp);
-    if ((rc = upload(&h->wpack, wp.data(), wp.size()))) return fail(rc);
+    if ((rc = upload(&h->wpack, wp.get(), (size_t)Np * Kp * (small ? 2 : 1)))) return fail(rc);
     if ((rc = upload(&h->colsum, colsum.data(), colsum.size()))) return fail(rc);
     if ((rc = upload(&h->c0, c0.data(), c0.size()))) return fail(rc);
     if ((rc = upload(&h->colscale, ws.data(), ws.size()))) return fail(rc);
