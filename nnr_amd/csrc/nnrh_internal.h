@@ -319,11 +319,11 @@ __host__ __device__ inline long long packed_off(int n, int k, int Kp) {
 // The same for the small-tile kernel, which loads operands straight into
 // registers: a piece is the operand of one MFMA, 16 consecutive columns x 64 K
 // bytes, one contiguous kilobyte, and the pieces of a column group follow each
-// other along K. (It reads the rows above 5 to 20 % slower: 197x3072x768 7.1 ->
-// 8.5 us, conv 8x56x56x64 3x3 7.3 -> 9.1. The kernels that stage tiles in LDS
-// lose as much on pieces: direct 3.6 -> 4.0 us, register-staged 34 -> 42,
-// pipelined 1562x768x1024 7.7 -> 8.0. So weights lie in memory both ways where
-// either kernel may run.)
+// other along K. (It reads the rows above 5 to 20 % slower: 197 rows, K = 3072, 768
+// columns 7.1 -> 8.5 us, 8 images of 56 x 56 x 64 3x3 7.3 -> 9.1. The kernels that
+// stage tiles in LDS lose as much on pieces: direct 3.6 -> 4.0 us, register-staged
+// 34 -> 42, pipelined 1562 rows, K = 768, 1024 columns 7.7 -> 8.0. So weights lie
+// in memory both ways where either kernel may run.)
 __host__ __device__ inline long long piece_off(int n, int k, int Kp) {
     return (long long)(n >> 4) * Kp * 16 + (long long)(k >> 6) * 1024 + (n & 15) * 64 + (k & 63);
 }

@@ -12,8 +12,9 @@
 // of K = 4608 in 36 dependent steps of load, barrier and MFMA (26 us). Here it
 // is 128 blocks of 16 waves whose every load is in flight at once (5.2 us; an
 // empty kernel takes 1.7). In a graph of one layer after another, weights from
-// the Infinity Cache: 196x256x2304 16.1 -> 3.7 us, 37x768x3072 18.5 -> 5.0,
-// 784x512x128 4.6 -> 2.9, 1x3072x768 7.7 -> 3.7, 1024x768x3072 19.7 -> 12.0.
+// the Infinity Cache, rows x columns x K: 196x256x2304 16.1 -> 3.7 us, 37x768x3072
+// 18.5 -> 5.0, 784x512x128 4.6 -> 2.9, 1x3072x768 7.7 -> 3.7, 1024x768x3072 19.7 ->
+// 12.0.
 // What is left is the L1's line rate on the operands, (1 / BM + 1 / BN) bytes
 // a multiply, and about 2.5 us of launch, first latency and drain.
 #include <cstdio>
@@ -215,8 +216,8 @@ __global__ __launch_bounds__(MAXW * 64) void qgemm_small_kernel(SmallArgs s, Gem
         for (int j = 0; j < NT; ++j) acc[i][j] = v4i{0, 0, 0, 0};
     // the two halves of a 128-byte line come with two loads; odd rows take
     // theirs in the other order, so that each load asks for both kinds of half
-    // (16 rows' equal halves cost the L1 twice the time: 512x768x3072 in
-    // 32x64 tiles 7.7 -> 6.8 us)
+    // (16 rows' equal halves cost the L1 twice the time: 512 rows, 768 columns,
+    // K = 3072 in 32x64 tiles 7.7 -> 6.8 us)
     const int odd = (frow & 1) * 64;
     struct Unit { v4i x[2][MT], w[2][NT]; };
     auto load_unit = [&](int u, Unit& d) {

@@ -1216,7 +1216,7 @@ def test_qconv1d(dev, case):
 
 @pytest.mark.parametrize("B,S,hidden,heads,scale", [
     (3, 37, 96, 4, 0.2),          # head size 24: two strided GEMMs + scaled softmax
-    (2, 160, 128, 2, 0.1),        # S > 128: the same
+    (2, 160, 128, 2, 0.1),        # S > 128: one kernel over the keys
     (2, 128, 768, 12, 0.125),     # head size 64, S <= 128: the fused kernel
     (3, 50, 128, 2, 0.3),         # fused, padded key rows and idle waves
     (2, 1, 64, 1, 0.5),           # fused, one token
@@ -1228,7 +1228,8 @@ def test_qconv1d(dev, case):
 ])
 def test_multihead_attention_f32(dev, B, S, hidden, heads, scale):
     """MultiHeadAttention (heads read and written in place; the fused fp32
-    MFMA kernel for head size 64 and S <= 128, two strided fp32 MFMA GEMMs
+    MFMA kernel for head size 64 and S <= 128, the one that walks the keys for
+    longer sequences and four other head sizes, two strided fp32 MFMA GEMMs
     over a (batch, head) grid and a scaled softmax otherwise) against float64
     numpy."""
     import torch
